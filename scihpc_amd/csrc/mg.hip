@@ -385,140 +385,9 @@ __global__ void __launch_bounds__(kBlock) k_coarse_solve(DLevel<T> G, const doub
   coarse_solve_block(G, Minv, neumann);
 }
 
-// the one-workgroup kernels below run with exactly kBlockThreads threads; a
-// constant stride keeps blockDim.x (a load from the dispatch packet) out of
-// their loops
-constexpr int kBlockThreads = 1024;
-// k_block_vcycle's dense coarsest solve gives each thread at most two rows
-static_assert(kMaxCoarse <= 2 * kBlockThreads, "coarsest rows exceed two per thread");
-
-// LDS-resident levels hold < 2^31 cells: 32-bit indices throughout
-template <typename T, int DIM, bool VAR>
-__device__ void block_sweep(const DLevel<T> &L, int first, int zero_guess) {
-  const int hx = (L.nx + 1) >> 1;
-  const int half = hx * L.ny * L.nz;
-  for (int pass = 0; pass < 2; ++pass) {
-    const int color = pass == 0 ? first : 1 - first;
-    for (int t = threadIdx.x; t < half; t += kBlockThreads) {
-      int i, j, k;
-      if constexpr (DIM == 2) {  // row j, colour cell t - j hx of it
-        j = (int)((unsigned)t / (unsigned)hx);
-        k = 0;
-        i = 2 * (t - j * hx) + ((j + color) & 1);
-        if (i >= L.nx) continue;
-      } else {
-        if (!color_cell(t, L.nx, L.ny, L.nz, color, i, j, k)) continue;
-      }
-      gs_cell<T, DIM, VAR, int>(L, i, j, k, pass == 0 ? zero_guess : 0);
-    }
-    __syncthreads();
-  }
-}
-
-// ---------------------------------------- one-workgroup coarse V-cycle
-// The latency-bound coarse levels (from the first level whose whole
-// remaining hierarchy fits in the workgroup's LDS) are cycled by a single
-// 1024-thread workgroup.  Every level's iterate, right-hand side and face
-// coefficients are staged into LDS once; each phase (one colour of a sweep,
-// restriction, dense coarsest solve, prolongation) is a strided loop over the
-// level followed by a workgroup barrier, so phases cost LDS latency rather
-// than global-memory round trips.  Only the top level's iterate is written
-// back.
-constexpr int kMaxBlockLevels = 12;
-
-template <typename T>
-struct BlockLevels {
-  DLevel<T> lv[kMaxBlockLevels];  // global views (read/write-back)
-  int ratio[kMaxBlockLevels];     // deg(l+1)/deg(l)
-  int off[kMaxBlockLevels];       // element offset of level l in LDS
-  int nlev;
-  int arrays;                     // arrays per level in LDS (2 or 2 + ndim)
-};
-
-// LDS view of block level l: global metadata, LDS arrays.  Built from the
-// extern __shared__ base on every use so the compiler keeps LDS (not flat)
-// addressing.
-template <typename T, bool VAR, int DIM>
-__device__ __forceinline__ DLevel<T> lds_view(const BlockLevels<T> *__restrict__ B, int l, T *smem) {
-  DLevel<T> v = B->lv[l];
-  T *base = smem + B->off[l];
-  const long n = v.n;
-  v.sol = base;
-  v.rhs = base + n;
-  if constexpr (VAR) {
-    v.cx = base + 2 * n;
-    v.cy = base + 3 * n;
-    if constexpr (DIM == 3) v.cz = base + 4 * n;
-  }
-  return v;
-}
-
-template <typename T, int DIM, bool VAR>
-__global__ void __launch_bounds__(kBlockThreads)
-    k_block_vcycle(const BlockLevels<T> *__restrict__ B, int nu1, int nu2, const double *__restrict__ Minv,
-                   int neumann, int dir, int zero_guess0, int load_top) {
-  extern __shared__ __align__(16) unsigned char smem_raw[];
-  T *smem = reinterpret_cast<T *>(smem_raw);
-  const int L = B->nlev;
-  for (int l = 0; l < L; ++l) {
-    const DLevel<T> g = B->lv[l];
-    const DLevel<T> S = lds_view<T, VAR, DIM>(B, l, smem);
-    for (long c = threadIdx.x; c < g.n; c += kBlockThreads) {
-      S.sol[c] = (l == 0 && load_top && !zero_guess0) ? g.sol[c] : T(0);
-      if (l == 0) S.rhs[c] = g.rhs[c];
-      if constexpr (VAR) {
-        const_cast<T *>(S.cx)[c] = g.cx[c];
-        const_cast<T *>(S.cy)[c] = g.cy[c];
-        if constexpr (DIM == 3) const_cast<T *>(S.cz)[c] = g.cz[c];
-      }
-    }
-  }
-  __syncthreads();
-  for (int l = 0; l < L - 1; ++l) {
-    const DLevel<T> F = lds_view<T, VAR, DIM>(B, l, smem);
-    const DLevel<T> G = lds_view<T, VAR, DIM>(B, l + 1, smem);
-    for (int s = 0; s < nu1; ++s) block_sweep<T, DIM, VAR>(F, 0, (l == 0 && s == 0) ? zero_guess0 : 0);
-    const int r = B->ratio[l];
-    for (int C = threadIdx.x; C < G.n; C += kBlockThreads) rr_cell<T, DIM, VAR, int>(F, G, r, C);
-    __syncthreads();
-  }
-  {  // dense coarsest solve, FP64, rows in registers
-    const DLevel<T> G = lds_view<T, VAR, DIM>(B, L - 1, smem);
-    const int n = (int)G.n;
-    double xr[2] = {0.0, 0.0};
-    double local = 0.0;
-    for (int q = 0; q < 2; ++q) {
-      const int row = threadIdx.x + q * kBlockThreads;
-      if (row < n) {
-        const double *m = Minv + (long)row * n;
-        double acc = 0.0;
-        for (int c = 0; c < n; ++c) acc += m[c] * double(G.rhs[c]);
-        xr[q] = acc;
-        local += acc;
-      }
-    }
-    const double tot = block_sum(local);
-    __shared__ double mean;
-    if (threadIdx.x == 0) mean = neumann ? tot / n : 0.0;
-    __syncthreads();
-    for (int q = 0; q < 2; ++q) {
-      const int row = threadIdx.x + q * kBlockThreads;
-      if (row < n) G.sol[row] = T(xr[q] - mean);
-    }
-    __syncthreads();
-  }
-  for (int l = L - 1; l > 0; --l) {
-    const DLevel<T> G = lds_view<T, VAR, DIM>(B, l, smem);
-    const DLevel<T> F = lds_view<T, VAR, DIM>(B, l - 1, smem);
-    const int r = B->ratio[l - 1];
-    for (int c = threadIdx.x; c < F.n; c += kBlockThreads) prolong_cell<T, DIM, int>(G, F, r, dir, c);
-    __syncthreads();
-    for (int s = 0; s < nu2; ++s) block_sweep<T, DIM, VAR>(F, 1, 0);
-  }
-  const DLevel<T> top = B->lv[0];
-  const DLevel<T> S0 = lds_view<T, VAR, DIM>(B, 0, smem);
-  for (long c = threadIdx.x; c < top.n; c += kBlockThreads) top.sol[c] = S0.sol[c];
-}
+}  // namespace scihpc
+#include "mg_block.hpp"
+namespace scihpc {
 
 // ---------------------------------------- fused 2-D fine-level kernels
 // A workgroup owns a TX x TY tile of a fine level and stages the iterate,
@@ -2215,6 +2084,10 @@ struct scihpc_mg {
   std::vector<Level<float>> f;  // FP32 hierarchy for the mixed path (lazy)
   std::vector<int> nocompat;
   double *Minv = nullptr;       // dense inverse of the (pinned) coarsest red-black operator
+  void *blk_pack[2] = {nullptr, nullptr};  // packs of the one-workgroup cycle, FP64 and FP32 (block_pack)
+  size_t blk_bytes[2] = {0, 0};
+  bool blk_ready[2] = {false, false};      // they match the operator
+  double *Minv_blk = nullptr;   // Minv transposed, the mean removal of the all-Neumann solve folded in
   double *Minv_ref = nullptr;   // same for the reference operator (differs for Dirichlet)
   double *partial = nullptr;    // per-block partial sums
   double *scal = nullptr;       // device scalars (S_*)
@@ -2232,8 +2105,6 @@ struct scihpc_mg {
                               // (SCIHPC_MG_FUSED_UPDATE=0 disables)
   int z3_chunk = 0;           // z planes per 3-D workgroup (0: chosen per level)
   float *rho0f = nullptr;     // FP32 copy of rho0 for the mixed V-cycle
-  void *blk_dev[2] = {nullptr, nullptr};   // device copies of BlockLevels<double>/<float>
-  std::vector<char> blk_host[2];           // last uploaded contents
   double *host_part = nullptr;             // pinned copy of the partial sums
   double *rho0 = nullptr;                  // level-0 density (MG layout) of the variable operator
   float *lfeat = nullptr, *lout = nullptr; // learned-guess features and network output
@@ -2504,64 +2375,180 @@ struct scihpc_mg {
     gs_color(l, 1 - first, 0);
   }
 
+  // ------------------------------------------- one-workgroup coarse cycle
+  // threads that patches of P rows need on a level
+  template <typename T>
+  static long block_patches(const Level<T> &l, int P) {
+    return (long)((l.nx + 1) / 2) * ((l.ny + P - 1) / P) * l.nz;
+  }
+  // workgroup size and rows a patch of a block cycle whose top level is lb;
+  // false when none holds it: the levels between the top and the coarsest
+  // need one pair of cells a thread at most
+  template <typename T>
+  bool block_shape(const std::vector<Level<T>> &lv, int lb, int &threads, int &rows) const {
+    constexpr bool dbl = sizeof(T) == 8;
+    static constexpr int shapes2[4][2] = {{512, 1}, {1024, 1}, {1024, 2}, {1024, 4}};
+    static constexpr int shapes3[3][2] = {{512, 1}, {512, 2}, {512, 4}};
+    for (int q = 0; q < (ndim == 3 ? 3 : dbl ? 3 : 4); ++q) {
+      const int nt = ndim == 3 ? shapes3[q][0] : shapes2[q][0], P = ndim == 3 ? shapes3[q][1] : shapes2[q][1];
+      if (lb < L - 1 && block_patches(lv[lb], P) > nt) continue;
+      if (lb + 1 < L - 1 && block_patches(lv[lb + 1], 1) > nt) continue;
+      threads = nt;
+      rows = P;
+      return true;
+    }
+    return false;
+  }
+  // descriptions of levels lb.. and their LDS layout; returns its bytes
+  template <typename T>
+  size_t block_layout(const std::vector<Level<T>> &lv, int lb, int threads, int rows, BlockArgs<T> &B,
+                      BlockGeo<T> *geo) const {
+    B.nlev = L - lb;
+    constexpr long e16 = 16 / sizeof(T);
+    long off = B.nlev * (long)(sizeof(BlockGeo<T>) / sizeof(T));
+    for (int i = 0; i < B.nlev; ++i) {
+      const auto &l = lv[lb + i];
+      BlockGeo<T> &g = geo[i];
+      g.nx = l.nx;
+      g.ny = l.ny;
+      g.nz = l.nz;
+      g.n = (int)l.n;
+      g.hx = (l.nx + 1) / 2;
+      g.pairs = (int)block_patches(l, 1);
+      g.ratio = i + 1 < B.nlev ? lv[lb + i + 1].deg / l.deg : 1;
+      const int P = i == 0 ? rows : 1;
+      g.sx = g.hx + 2;
+      g.sz = g.sx * ((l.ny + P - 1) / P * P + 2);
+      g.xc = ndim == 3 ? g.sz * (l.nz + 2) : g.sz;
+      g.ihx = 1.0f / float(g.hx);
+      g.iny = 1.0f / float(g.ny);
+      g.spare = 0;
+      g.co = g.bo = 0;
+      if (i > 0 && i + 1 < B.nlev) {
+        g.co = (int)off;
+        off += (long)(ndim == 3 ? block_fields<3>() : block_fields<2>()) * g.pairs;
+      }
+    }
+    off = (off + e16 - 1) / e16 * e16;
+    B.pack16 = (int)(off / e16);
+    B.xo16 = (int)(off / e16);
+    for (int i = 0; i < B.nlev; ++i) {
+      geo[i].xo = (int)off;
+      off += 2L * geo[i].xc;
+    }
+    off = (off + e16 - 1) / e16 * e16;
+    B.xn16 = (int)(off / e16) - B.xo16;
+    B.ro = (int)off;
+    if (B.nlev > 1) off += 2L * geo[0].pairs;
+    for (int i = 1; i + 1 < B.nlev; ++i) {
+      geo[i].bo = (int)off;
+      off += 2L * geo[i].pairs;
+    }
+    off = (off + e16 - 1) / e16 * e16;
+    B.dense = (int)(off * (long)sizeof(T));
+    B.nc = (int)lv[L - 1].n;
+    const int nrp = (B.nc + 1) / 2;
+    B.ld = 2 * nrp;
+    B.split = std::max(1, std::min(kBlockSplit, threads / nrp));
+    B.per = (int)ceil_div(B.nc, B.split);
+    return off * sizeof(T) + sizeof(double) * 2 * nrp * (1 + B.split);
+  }
   // first level cycled by the one-workgroup LDS kernel (L when even the
-  // coarsest level does not fit the LDS budget)
+  // coarsest level does not fit the LDS budget).  Level 0 itself is taken up
+  // to 4096 cells: the FCG iteration of larger ones is shorter with the tiled
+  // level-0 kernels, which carry the vector updates.
   template <typename T>
   int block_level(const std::vector<Level<T>> &lv) const {
-    const long bpc = (long)sizeof(T) * (2 + (variable ? ndim : 0));
-    const long budget = lds_max - 2048;
-    long used = 0;
     int lb = L;
     for (int l = L - 1; l >= 0 && l >= L - kMaxBlockLevels; --l) {
-      used += lv[l].n * bpc;
-      if (used > budget || lv[l].n > block_max) break;
+      int threads, rows;
+      if (lv[l].n > block_max || !block_shape(lv, l, threads, rows) || (l == 0 && lv[l].n > 4096)) break;
+      BlockArgs<T> B;
+      BlockGeo<T> geo[kMaxBlockLevels];
+      if (block_layout(lv, l, threads, rows, B, geo) > (size_t)lds_max) break;
       lb = l;
     }
     return lb;
   }
 
+  template <typename T, int DIM, int P, int NT>
+  void block_launch(const BlockArgs<T> &B, size_t bytes) {
+    if (bytes > 65536)
+      SCIHPC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_block_vcycle<T, DIM, P, NT>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+    k_block_vcycle<T, DIM, P, NT><<<1, NT, bytes, stream>>>(B);
+    SCIHPC_CHECK_LAUNCH();
+  }
+  // the block cycle's pack (level descriptions and records) on the device,
+  // rebuilt on the first cycle after the operator changed
+  template <typename T>
+  void block_pack(const std::vector<Level<T>> &lv, int lb, const BlockArgs<T> &B, const BlockGeo<T> *geo) {
+    const int slot = std::is_same<T, double>::value ? 0 : 1;
+    const size_t bytes = 16 * (size_t)B.pack16;
+    if (blk_bytes[slot] < bytes) {
+      if (blk_pack[slot]) SCIHPC_HIP(hipFree(blk_pack[slot]));
+      blk_pack[slot] = nullptr;
+      blk_bytes[slot] = 0;
+      SCIHPC_HIP(hipMalloc(&blk_pack[slot], bytes));
+      blk_bytes[slot] = bytes;
+    }
+    SCIHPC_HIP(hipMemcpyAsync(blk_pack[slot], geo, sizeof(BlockGeo<T>) * B.nlev, hipMemcpyHostToDevice, stream));
+    for (int i = 1; i + 1 < B.nlev; ++i) {
+      T *out = static_cast<T *>(blk_pack[slot]) + geo[i].co;
+      const unsigned nb = ceil_div(geo[i].pairs, kBlock);
+      if (ndim == 2) k_block_pack<T, 2><<<nb, kBlock, 0, stream>>>(view(lv[lb + i]), geo[i].hx, geo[i].pairs, out);
+      else k_block_pack<T, 3><<<nb, kBlock, 0, stream>>>(view(lv[lb + i]), geo[i].hx, geo[i].pairs, out);
+      SCIHPC_CHECK_LAUNCH();
+    }
+    SCIHPC_HIP(hipStreamSynchronize(stream));  // geo is the caller's
+    blk_ready[slot] = true;
+  }
   template <typename T>
   void block_cycle(std::vector<Level<T>> &lv, int lb, int nu1, int nu2, int zero_guess0, int load_top) {
-    BlockLevels<T> B;
-    std::memset(&B, 0, sizeof(B));
-    B.nlev = L - lb;
-    B.arrays = 2 + (variable ? ndim : 0);
-    long off = 0;
-    for (int i = 0; i < B.nlev; ++i) {
-      B.lv[i] = view(lv[lb + i]);
-      B.ratio[i] = i + 1 < B.nlev ? lv[lb + i + 1].deg / lv[lb + i].deg : 1;
-      B.off[i] = (int)off;
-      off += lv[lb + i].n * B.arrays;
-    }
-    const size_t bytes = sizeof(T) * off;
-    const int neu = bc == SCIHPC_MG_NEUMANN, dir = bc == SCIHPC_MG_DIRICHLET;
-    // the metadata lives in device memory (a by-value kernel argument indexed
-    // by level would be copied to scratch); re-uploaded only when it changes
+    BlockArgs<T> B;
+    BlockGeo<T> geo[kMaxBlockLevels];
+    int threads = 0, rows = 0;
+    SCIHPC_REQUIRE(block_shape(lv, lb, threads, rows), "internal: block cycle shape");
+    const size_t bytes = block_layout(lv, lb, threads, rows, B, geo);
     const int slot = std::is_same<T, double>::value ? 0 : 1;
-    if (!blk_dev[slot]) SCIHPC_HIP(hipMalloc(&blk_dev[slot], sizeof(BlockLevels<double>)));
-    if (blk_host[slot].size() != sizeof(B) || std::memcmp(blk_host[slot].data(), &B, sizeof(B)) != 0) {
-      blk_host[slot].assign(reinterpret_cast<const char *>(&B), reinterpret_cast<const char *>(&B) + sizeof(B));
-      SCIHPC_HIP(hipMemcpyAsync(blk_dev[slot], blk_host[slot].data(), sizeof(B), hipMemcpyHostToDevice, stream));
-      SCIHPC_HIP(hipStreamSynchronize(stream));
-    }
-    const BlockLevels<T> *Bd = static_cast<const BlockLevels<T> *>(blk_dev[slot]);
-#define SCIHPC_BLOCK(D, V)                                                                                  \
-  do {                                                                                                      \
-    if (bytes > 65536)                                                                                      \
-      SCIHPC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_block_vcycle<T, D, V>),             \
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));              \
-    k_block_vcycle<T, D, V><<<1, kBlockThreads, bytes, stream>>>(Bd, nu1, nu2, Minv, neu, dir, zero_guess0, \
-                                                                  load_top);                                \
-  } while (0)
+    if (!blk_ready[slot]) block_pack(lv, lb, B, geo);
+    const DLevel<T> v = view(lv[lb]);
+    B.top = geo[0];
+    B.cx = v.cx;
+    B.cy = v.cy;
+    B.cz = v.cz;
+    B.ax = v.ax;
+    B.ay = v.ay;
+    B.az = v.az;
+    B.dconst = v.dconst;
+    B.wx = v.wx;
+    B.wy = v.wy;
+    B.wz = v.wz;
+    B.dirichlet = v.dirichlet;
+    B.rbwall = v.rbwall;
+    B.rhs = v.rhs;
+    B.sol_in = B.sol_out = v.sol;
+    B.pack = static_cast<const BlockWords *>(blk_pack[slot]);
+    B.Mt = Minv_blk;
+    B.dir = bc == SCIHPC_MG_DIRICHLET;
+    B.nu1 = nu1;
+    B.nu2 = nu2;
+    B.zero_top = (load_top && !zero_guess0) ? 0 : 1;
     if (ndim == 2) {
-      if (variable) SCIHPC_BLOCK(2, true);
-      else SCIHPC_BLOCK(2, false);
+      if constexpr (sizeof(T) == 4) {
+        if (rows == 4) {
+          block_launch<T, 2, 4, 1024>(B, bytes);
+          return;
+        }
+      }
+      if (threads == 512) block_launch<T, 2, 1, 512>(B, bytes);
+      else if (rows == 1) block_launch<T, 2, 1, 1024>(B, bytes);
+      else block_launch<T, 2, 2, 1024>(B, bytes);
     } else {
-      if (variable) SCIHPC_BLOCK(3, true);
-      else SCIHPC_BLOCK(3, false);
+      if (rows == 1) block_launch<T, 3, 1, 512>(B, bytes);
+      else if (rows == 2) block_launch<T, 3, 2, 512>(B, bytes);
+      else block_launch<T, 3, 4, 512>(B, bytes);
     }
-#undef SCIHPC_BLOCK
-    SCIHPC_CHECK_LAUNCH();
   }
 
   // V(nu1,nu2) on hierarchy `lv`, in place on lv[0].sol.  Fine 2-D levels
@@ -2919,6 +2906,23 @@ struct scihpc_mg {
       }
     }
     SCIHPC_HIP(hipMemcpyAsync(dst, Inv.data(), sizeof(double) * n * n, hipMemcpyHostToDevice, stream));
+    std::vector<double> Mt;
+    if (rb) {
+      // for the block cycle: column c of Inv as row c, less its mean for
+      // all-Neumann operators (x - mean(x) = (Inv - 1 w^T) b, w the column means)
+      // rows padded to an even length
+      const int ld = (n + 1) / 2 * 2;
+      Mt.assign((size_t)n * ld, 0.0);
+      for (int c = 0; c < n; ++c) {
+        double w = 0.0;
+        if (bc == SCIHPC_MG_NEUMANN) {
+          for (int r = 0; r < n; ++r) w += Inv[(size_t)r * n + c];
+          w /= n;
+        }
+        for (int r = 0; r < n; ++r) Mt[(size_t)c * ld + r] = Inv[(size_t)r * n + c] - w;
+      }
+      SCIHPC_HIP(hipMemcpyAsync(Minv_blk, Mt.data(), sizeof(double) * n * ld, hipMemcpyHostToDevice, stream));
+    }
     SCIHPC_HIP(hipStreamSynchronize(stream));
   }
 
@@ -2993,6 +2997,7 @@ struct scihpc_mg {
     SCIHPC_HIP(hipStreamSynchronize(stream));
     if (!f.empty())
       for (int l = 0; l < L; ++l) refresh_fp32_faces(l);
+    blk_ready[0] = blk_ready[1] = false;
     build_coarse_inverse(true, Minv);  // Neumann: Minv_ref aliases Minv
   }
 
@@ -3755,6 +3760,8 @@ extern "C" int scihpc_mg_create(int ndim, int nx, int ny, int nz, double dx, dou
       }
       h->Minv = dalloc<double>((long)std::min<long>(h->d.back().n, kMaxCoarse) *
                                std::min<long>(h->d.back().n, kMaxCoarse), h->stream);
+      h->Minv_blk = dalloc<double>((long)std::min<long>(h->d.back().n, kMaxCoarse) *
+                                   (std::min<long>(h->d.back().n, kMaxCoarse) + 1), h->stream);
       h->partial = dalloc<double>(8 * ((long)ceil_div(h->d[0].n, kBlock) + 64), h->stream);
       h->partial2 = dalloc<double>(4 * ((long)ceil_div(h->d[0].n, (long)kBlock * kBlock) + 64), h->stream);
       SCIHPC_HIP(hipHostMalloc((void **)&h->host_part,
@@ -3819,10 +3826,11 @@ extern "C" int scihpc_mg_destroy(scihpc_mg *h) {
   }
   if (h->Minv_ref != h->Minv) fr(h->Minv_ref);
   fr(h->Minv);
+  fr(h->Minv_blk);
+  fr(h->blk_pack[0]);
+  fr(h->blk_pack[1]);
   fr(h->partial);
   fr(h->partial2);
-  fr(h->blk_dev[0]);
-  fr(h->blk_dev[1]);
   if (h->host_part) (void)hipHostFree(h->host_part);
   fr(h->fx_);
   fr(h->fr_);
