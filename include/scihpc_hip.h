@@ -465,8 +465,9 @@ enum { SCIHPC_LS_WENO5 = 0, SCIHPC_LS_UCCD = 1 };
 SCIHPC_API int scihpc_ls_set_scheme(scihpc_ls *h, int scheme);
 /* How the CCD/UCCD line systems are solved (the twin back substitution of
  * matrix_solver.cpp:58-83 on the factorised coefficients of twin_dec,
- * :21-56).  partitioned = 0 (the default): one thread per line in the
- * reference's order, bit-identical to it.  partitioned = 1: every line cut
+ * :21-56).  partitioned = 0 (the default): the values of the reference's
+ * sequential order, bit for bit (lines are swept in segments that start from
+ * overlapping warm-ups, each checked against its neighbour's final state).  partitioned = 1: every line cut
  * into segments that sweep in parallel and exchange their incoming states
  * through 2x2 segment propagators, then sweep again from the true states
  * with the reference's arithmetic; the results differ from the sequential

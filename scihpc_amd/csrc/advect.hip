@@ -14,6 +14,8 @@
 // are never written, as in the reference.
 #include <algorithm>
 #include <cmath>
+#include <cstring>
+#include <type_traits>
 #include <utility>
 #include <vector>
 
@@ -944,6 +946,394 @@ __global__ void __launch_bounds__(64) k_twin_line(Grid g, int nsys, LineCoefs co
   }
 }
 
+// ---- the sequential sweeps' values without their chain of 2 n steps.
+// Both sweeps contract (|eig M_i| <= 0.25 and |eig D_i^-1 N_i| <= 0.65
+// inside a line), and not only in exact arithmetic: two forward (backward)
+// sweeps over the same right-hand sides that start from different states
+// round to the same bits after some steps.  So every line is cut into
+// segments, one thread each: a segment starts `warm` positions early from a
+// zero state (or, if that reaches the line's end, from the exact one), sweeps
+// up to its own first position, then sweeps its own positions in place.
+// Whether the incoming state it arrived at equals the neighbour's final value
+// is checked: if all do the result is the sequential sweep's, bit for bit.  If one is not (a chance below 1e-6 a segment with the warm
+// lengths below, measured on random and smooth data; always where the
+// right-hand side is exactly 0 over a whole warm-up), or if a value is not
+// finite or nearly denormal, the workgroup forms its right-hand sides again and
+// sweeps its lines end to end, one thread each, with IEEE quotients.
+//
+// A workgroup holds LINES whole lines in LDS, UCCD's two systems side by
+// side, and does everything from the field to the derivatives: right-hand
+// sides, sweeps, selection.  The factorised coefficients repeat along the
+// line from about the 27th position on with a period of at most 3 (their
+// elimination reaches a fixed point of the rounding), so a table of about 30
+// rows serves any line; the host checks the period.  The backward sweep's
+// quotients by the rows' determinants are formed from the stored reciprocal
+// with two exact-remainder corrections, which rounds them correctly
+// (Markstein: after the first correction the quotient is within an ulp, and
+// the second, with the reciprocal correctly rounded, gives the nearest);
+// only the sign of a zero may differ.  Segment lengths are odd, so the 64
+// lanes of a wavefront (LINES lines x 64 / LINES segments) read different
+// banks.
+// What bounds it: the instructions a lone wavefront issues for about 240
+// steps forward and 230 backward (instead of 2 x 1030), and LDS: whole lines
+// leave one workgroup a CU, so 389 workgroups run as two rounds.  Measured at
+// 1024 x 512: 91 us, where right-hand sides, one thread a line and selection
+// took 11.7 + 383 + 7.2 us in three launches; a UCCD TVD-RK3 step 1.25 ->
+// 0.34 ms.  Lines that do not fit LDS (over about 4700 points) keep the three
+// passes.
+struct TwinTable {
+  const double *row[3][2];           // [axis][system]: rows of kTwinRow values
+  int start[3][2], period[3][2], rows[3][2];
+};
+constexpr int kTwinRow = 14;         // a0 b0 aa0 bb0 | a2 b2 aa2 bb2 | a1 b1 aa1 bb1 | den 1/den
+constexpr int kTwinRowsMax = 96;
+struct TwinPlan {
+  int waves;                         // wavefronts a system
+  int len[3], segs[3];               // positions a segment (odd), segments
+  int cap;                           // LDS doubles of one array
+  int blocks[3];                     // workgroups of each axis
+};
+// warm-up positions [CCD, UCCD upwind, UCCD downwind]
+__device__ constexpr int kTwinWarmF[3] = {102, 210, 48}, kTwinWarmB[3] = {102, 48, 192};
+
+// row of the table for position i
+__device__ __forceinline__ int twin_row(int i, int n, int start, int period, int rows) {
+  return i == n - 1 ? rows - 1 : i < start ? i : start + (i - start) % period;
+}
+
+__device__ __forceinline__ double twin_quot(double a, double d, double r) {
+#pragma clang fp contract(off)
+  double q = a * r;
+  q = __builtin_fma(__builtin_fma(-d, q, a), r, q);
+  return __builtin_fma(__builtin_fma(-d, q, a), r, q);
+}
+
+// 0 < |x| < 2^-862 (but for the last denormals): there twin_quot's remainders
+// are no longer exact
+__device__ __forceinline__ bool twin_tiny(double x) {
+  return ((unsigned)__double2hiint(x) << 1) - 1u < ((1023u - 862u) << 21) - 1u;
+}
+
+template <int LINES, bool UP>
+__global__ void __launch_bounds__(512)  // two systems, at most four wavefronts each
+    k_twin_seg(Grid g, const double *__restrict__ f, const double *__restrict__ u, const double *__restrict__ v,
+               const double *__restrict__ w, TwinTable tb, TwinPlan pl, double *__restrict__ d1x,
+               double *__restrict__ d1y, double *__restrict__ d1z, double *__restrict__ d2x,
+               double *__restrict__ d2y, double *__restrict__ d2z) {
+#pragma clang fp contract(off)
+  constexpr int NS = UP ? 2 : 1;
+  extern __shared__ __align__(16) double twin_lds[];
+  // neighbouring line groups on one XCD: they share the field's cache lines
+  int b = blockIdx.x;
+  if (gridDim.x % 8 == 0) b = (b % 8) * (int)(gridDim.x / 8) + b / 8;
+  int a = 0;
+  while (a < 2 && b >= pl.blocks[a]) b -= pl.blocks[a++];
+  const int n = g.N[a], len = pl.len[a], segs = pl.segs[a];
+  const long st = g.s[a];
+  const int tid = threadIdx.x, nt = blockDim.x;
+  const int sys = UP ? tid / (64 * pl.waves) : 0;
+  const int ts = tid - sys * 64 * pl.waves;
+  const int ln = ts % LINES, seg = ts / LINES;
+  double *const S = twin_lds + (size_t)sys * 2 * pl.cap, *const SS = S + pl.cap;
+  double *const tab = twin_lds + (size_t)(UP ? 4 : 3) * pl.cap;
+
+  // The workgroup's cells, kTwinBatch a thread at a time so that their loads
+  // are in flight together: get(address) of each, then put(value, LDS index,
+  // address, line exists).  Neighbouring lanes take neighbouring cells in
+  // memory: along the line where it is contiguous, else across the lines.
+  constexpr int kTwinBatch = 16;
+  const long line0 = (long)b * LINES, lines = (long)g.N[(a + 1) % 3] * g.N[(a + 2) % 3];
+  const bool along = st == 1;
+  long own_base = 0;
+  const bool own_ok = line_base(g, a, line0 + tid % LINES, own_base);
+  const int hop = along ? nt : nt / LINES;
+  const long hop_c = hop * st;
+  auto cells = [&](auto get, auto put) {
+    for (int i0 = along ? tid : tid / LINES; i0 < n; i0 += (along ? kTwinBatch / LINES : kTwinBatch) * hop) {
+      double v[kTwinBatch];
+      const long c0 = (along ? line0 * n : own_base) + i0 * st;
+#pragma unroll
+      for (int q = 0; q < kTwinBatch; ++q) {
+        const int i = i0 + (along ? q / LINES : q) * hop;
+        const bool ok = i < n && (along ? line0 + q % LINES < lines : own_ok);
+        const long c = c0 + (along ? (q % LINES) * n + (q / LINES) * hop : q * hop_c);
+        v[q] = ok ? get(c) : 0.0;
+      }
+#pragma unroll
+      for (int q = 0; q < kTwinBatch; ++q) {
+        const int i = i0 + (along ? q / LINES : q) * hop, l = along ? q % LINES : tid % LINES;
+        const bool ok = along ? line0 + q % LINES < lines : own_ok;
+        const long c = c0 + (along ? (q % LINES) * n + (q / LINES) * hop : q * hop_c);
+        if (i < n) put(v[q], i, l, c, ok);
+      }
+    }
+  };
+  // the right-hand sides, exactly: compact_rhs from the field in memory
+  auto fill = [&]() {
+    cells([](long) { return 0.0; }, [&](double, int i, int l, long c, bool ok) {
+      double s0 = 0.0, ss0 = 0.0, s1 = 0.0, ss1 = 0.0;
+      if (ok) {
+        const double *line = f + (c - (long)i * st);
+        if (UP) {
+          compact_rhs<1>(line, st, n, g.h[a], i, s0, ss0);
+          s1 = s0;
+          ss1 = ss0;
+          if (i > 0 && i < n - 1) compact_rhs<2>(line, st, n, g.h[a], i, s1, ss1);  // the ends are the upwind ones
+        } else {
+          compact_rhs<0>(line, st, n, g.h[a], i, s0, ss0);
+        }
+      }
+      double *p = twin_lds + i * LINES + l;
+      p[0] = s0;
+      p[pl.cap] = ss0;
+      if (UP) {
+        p[2 * pl.cap] = s1;
+        p[3 * pl.cap] = ss1;
+      }
+    });
+  };
+  for (int y = 0; y < NS; ++y)
+    for (int t = tid; t < kTwinRow * tb.rows[a][y]; t += nt) tab[y * kTwinRow * kTwinRowsMax + t] = tb.row[a][y][t];
+  {
+    // The same values from LDS: the field goes to the last array (UCCD: the
+    // downwind f'' array, which gets its values from the upwind one), then
+    // every right-hand side to its own.  The
+    // divisions by h are twin_quot's (a value that is not finite there ends in
+    // the exact path below).
+    double *const F = twin_lds + (size_t)(UP ? 3 : 2) * pl.cap;
+    cells([&](long c) { return f[c]; }, [&](double z, int i, int l, long, bool) { F[i * LINES + l] = z; });
+    __syncthreads();
+    const double h = g.h[a], rh = 1.0 / h;
+    auto rhs = [&](int l, int i, double &s0, double &ss0, double &s1) {
+      const double *z = F + l;
+      if (i == 0 || i == n - 1) {  // the one-sided ends
+        const int o = i == 0 ? 0 : (n - 1) * LINES, d = i == 0 ? LINES : -LINES;
+        const double x0 = z[o], x1 = z[o + d], x2 = z[o + 2 * d];
+        const double e = -3.5 * x0 + 4.0 * x1 + -0.5 * x2, ee = 9.0 * x0 + -12.0 * x1 + 3.0 * x2;
+        s0 = s1 = twin_quot(i == 0 ? e : -e, h, rh);
+        ss0 = twin_quot(twin_quot(ee, h, rh), h, rh);
+        return;
+      }
+      const double c3 = -0.06096119008109, c2 = 1.99692238016218, c1 = -1.93596119008109;
+      const double m = z[(i - 1) * LINES], c = z[i * LINES], q = z[(i + 1) * LINES];
+      if (UP) {
+        s0 = twin_quot(c1 * m + c2 * c + c3 * q, h, rh);
+        s1 = twin_quot(-(c3 * m + c2 * c + c1 * q), h, rh);
+      } else {
+        s0 = twin_quot(15.0 / 16.0 * (q - m), h, rh);
+      }
+      ss0 = twin_quot(twin_quot(3.0 * m - 6.0 * c + 3.0 * q, h, rh), h, rh);
+    };
+    const int m = n * LINES;  // cell t of these: position t / LINES, line t % LINES
+#pragma unroll 4
+    for (int t = tid; t < m; t += nt) {
+      double s0, ss0, s1 = 0.0;
+      rhs(t % LINES, t / LINES, s0, ss0, s1);
+      twin_lds[t] = s0;
+      twin_lds[pl.cap + t] = ss0;
+      if (UP) twin_lds[2 * pl.cap + t] = s1;
+    }
+    if (UP) {
+      __syncthreads();
+#pragma unroll 4
+      for (int t = tid; t < m; t += nt) twin_lds[3 * pl.cap + t] = twin_lds[pl.cap + t];
+    }
+  }
+  __syncthreads();
+
+  const double *const T = tab + sys * kTwinRow * kTwinRowsMax;
+  const int start = tb.start[a][sys], period = tb.period[a][sys], rows = tb.rows[a][sys];
+  const int kind = UP ? 1 + sys : 0;
+  const int lo = seg * len, hi = min(n, lo + len);
+  const bool on = seg < segs && lo < n;
+  int bad = 0;  // a state that does not match, or a value that twin_quot may not round exactly
+  auto at = [&](int i) { return i * LINES + ln; };
+
+  // A step's cost is the instructions a lone wavefront issues for it, so
+  // where the rows repeat (from `start` on; the period divides kTwinUnroll)
+  // a thread keeps its kTwinUnroll rows in registers and runs blocks of that
+  // many steps with nothing but the values to load; single steps with the
+  // row looked up are left for the line's beginning and the remainders.
+  constexpr int kTwinUnroll = 6;
+  auto frow = [&](const double *c, double vs, double vss, double &p, double &q) {
+    const double x = vs - (c[0] * p + c[1] * q);
+    const double y = vss - (c[2] * p + c[3] * q);
+    p = x;
+    q = y;
+  };
+  auto fstep = [&](int i, int r, bool keep, double &p, double &q) {
+    frow(T + r * kTwinRow, S[at(i)], SS[at(i)], p, q);
+    if (keep) {
+      S[at(i)] = p;
+      SS[at(i)] = q;
+    }
+  };
+  auto forward = [&](int i, int end, bool keep, double &p, double &q) {
+#pragma unroll 2
+    for (; i < min(end, start); ++i) fstep(i, i == n - 1 ? rows - 1 : i, keep, p, q);
+    if (i >= end) return;
+    const int stop = min(end, n - 1);
+    int ph = (int)((unsigned)(i - start) % (unsigned)period);
+    if (i + kTwinUnroll <= stop) {
+      double c[kTwinUnroll][4];
+      int w = ph;
+#pragma unroll
+      for (int k = 0; k < kTwinUnroll; ++k) {
+#pragma unroll
+        for (int e = 0; e < 4; ++e) c[k][e] = T[(start + w) * kTwinRow + e];
+        w = w + 1 == period ? 0 : w + 1;
+      }
+      do {
+        double vs[kTwinUnroll], vss[kTwinUnroll];
+#pragma unroll
+        for (int k = 0; k < kTwinUnroll; ++k) {
+          vs[k] = S[at(i + k)];
+          vss[k] = SS[at(i + k)];
+        }
+#pragma unroll
+        for (int k = 0; k < kTwinUnroll; ++k) {
+          frow(c[k], vs[k], vss[k], p, q);
+          if (keep) {
+            S[at(i + k)] = p;
+            SS[at(i + k)] = q;
+          }
+        }
+        i += kTwinUnroll;
+      } while (i + kTwinUnroll <= stop);
+    }
+    for (; i < end; ++i) {
+      fstep(i, i == n - 1 ? rows - 1 : start + ph, keep, p, q);
+      ph = ph + 1 == period ? 0 : ph + 1;
+    }
+  };
+  double p = 0.0, q = 0.0, pin, qin;
+  if (on) {
+    const int i = max(lo - kTwinWarmF[kind], 1);
+    if (i == 1 || seg == 0) {
+      p = S[at(0)];
+      q = SS[at(0)];
+    }
+    forward(i, lo, false, p, q);
+  }
+  pin = p;
+  qin = q;
+  __syncthreads();
+  if (on) forward(max(lo, 1), hi, true, p, q);
+  __syncthreads();
+  if (on && seg > 0)
+    bad |= S[at(lo - 1)] != pin || SS[at(lo - 1)] != qin;
+  // backward, the same way; the closure at n - 1 is not one of these steps
+  // (kind of quotient: std::true_type IEEE, std::false_type twin_quot).
+  auto solve2 = [&](auto ieee, const double *c, double si, double ti, double &x, double &y) {
+    const double nx = -(c[5] * ti - c[7] * si), ny = c[4] * ti - c[6] * si;
+    x = ieee ? nx / c[8] : twin_quot(nx, c[8], c[9]);
+    y = ieee ? ny / c[8] : twin_quot(ny, c[8], c[9]);
+  };
+  auto brow = [&](auto ieee, const double *c, double vs, double vss, double &x, double &y) {
+    solve2(ieee, c, vs - (c[0] * x + c[1] * y), vss - (c[2] * x + c[3] * y), x, y);
+  };
+  auto bstep = [&](auto ieee, int i, int r, bool keep, double &x, double &y) {
+    brow(ieee, T + r * kTwinRow + 4, S[at(i)], SS[at(i)], x, y);
+    if (keep) {
+      bad |= twin_tiny(x) || twin_tiny(y);
+      S[at(i)] = x;
+      SS[at(i)] = y;
+    }
+  };
+  auto backward = [&](auto ieee, int i, int end, bool keep, double &x, double &y) {
+    const int stop = max(end, start);
+    if (i >= stop) {
+      int ph = (int)((unsigned)(i - start) % (unsigned)period);
+      if (i - kTwinUnroll + 1 >= stop) {
+        double c[kTwinUnroll][10];
+        int w = ph;
+#pragma unroll
+        for (int k = 0; k < kTwinUnroll; ++k) {
+#pragma unroll
+          for (int e = 0; e < 10; ++e) c[k][e] = T[(start + w) * kTwinRow + 4 + e];
+          w = w == 0 ? period - 1 : w - 1;
+        }
+        do {
+          double vs[kTwinUnroll], vss[kTwinUnroll];
+#pragma unroll
+          for (int k = 0; k < kTwinUnroll; ++k) {
+            vs[k] = S[at(i - k)];
+            vss[k] = SS[at(i - k)];
+          }
+#pragma unroll
+          for (int k = 0; k < kTwinUnroll; ++k) {
+            brow(ieee, c[k], vs[k], vss[k], x, y);
+            if (keep) {
+              bad |= twin_tiny(x) || twin_tiny(y);
+              S[at(i - k)] = x;
+              SS[at(i - k)] = y;
+            }
+          }
+          i -= kTwinUnroll;
+        } while (i - kTwinUnroll + 1 >= stop);
+      }
+      for (; i >= stop; --i) {
+        bstep(ieee, i, start + ph, keep, x, y);
+        ph = ph == 0 ? period - 1 : ph - 1;
+      }
+    }
+#pragma unroll 2
+    for (; i >= end; --i) bstep(ieee, i, i, keep, x, y);
+  };
+  double x = 0.0, y = 0.0, xin, yin;
+  if (on) {
+    int i = min(hi - 1 + kTwinWarmB[kind], n - 1);
+    if (i == n - 1) {  // the closure
+      solve2(std::false_type(), T + (rows - 1) * kTwinRow + 4, S[at(i)], SS[at(i)], x, y);
+      --i;
+    }
+    backward(std::false_type(), i, hi, false, x, y);
+  }
+  xin = x;
+  yin = y;
+  __syncthreads();
+  if (on) {
+    if (hi == n) {
+      S[at(n - 1)] = x;
+      SS[at(n - 1)] = y;
+    }
+    backward(std::false_type(), min(hi - 1, n - 2), lo, true, x, y);
+    bad |= !(fabs(x) < __builtin_inf()) || !(fabs(y) < __builtin_inf());
+  }
+  __syncthreads();
+  if (on && hi < n)
+    bad |= S[at(hi)] != xin || SS[at(hi)] != yin;
+  if (__syncthreads_or(bad)) {  // one thread a line from end to end
+    fill();
+    __syncthreads();
+    if (seg == 0) {
+      p = S[at(0)];
+      q = SS[at(0)];
+      forward(1, n, true, p, q);
+      solve2(std::true_type(), T + (rows - 1) * kTwinRow + 4, p, q, x, y);
+      S[at(n - 1)] = x;
+      SS[at(n - 1)] = y;
+      backward(std::true_type(), n - 2, 0, true, x, y);
+    }
+    __syncthreads();
+  }
+
+  // the derivatives, as k_compact_select forms them
+  const double *vel = a == 0 ? u : a == 1 ? v : w;
+  double *const d1 = a == 0 ? d1x : a == 1 ? d1y : d1z, *const d2 = a == 0 ? d2x : a == 1 ? d2y : d2z;
+  cells([&](long c) { return UP ? vel[c] : 0.0; }, [&](double vc, int i, int l, long c, bool ok) {
+    if (!ok) return;
+    const double *z = twin_lds + i * LINES + l;
+    if (UP) {
+      d1[c] = vc > 0 ? z[0] : z[2 * pl.cap];
+      if (d2) d2[c] = 0.5 * (z[pl.cap] + z[3 * pl.cap]);
+    } else {
+      d1[c] = z[0];
+      if (d2) d2[c] = z[pl.cap];
+    }
+  });
+}
+
 // The twin sweeps partitioned along the line, for the latency of the
 // recurrence: k_twin_line's chain of 2 n dependent steps per line (with two
 // FP64 divisions per backward step) on a few thousand threads becomes about
@@ -1630,6 +2020,13 @@ struct scihpc_ls {
   int twin_lines = 0, twin_len = 0;
   double *carry = nullptr;
   bool twin_partitioned = false;
+  // segmented sequential sweeps (k_twin_seg): coefficient rows [axis][CCD,
+  // UCCD up, UCCD down], and the rows' repetition along a line; seg_ok when
+  // every axis has one
+  double *seg_rows[3][3] = {};
+  int seg_start[3][3] = {}, seg_period[3][3] = {}, seg_count[3][3] = {};
+  bool seg_ok = false;
+  bool seg_lds_set[2][3] = {};  // k_twin_seg<LINES, UP> has been allowed its dynamic LDS, [UP][LINES / 2]
   int lds_max = 65536;      // LDS bytes a workgroup may hold on this device
   size_t twin_lds_set = 0;  // dynamic LDS the partitioned kernels have been allowed
 
@@ -1640,6 +2037,7 @@ struct scihpc_ls {
       const std::vector<double> cc = compact_coefficients(0, n, g.h[a]);
       const std::vector<double> cu = compact_coefficients(1, n, g.h[a]);
       const std::vector<double> cd = compact_coefficients(2, n, g.h[a]);
+      seg_ok = (a == 0 || seg_ok) && seg_table(a, 0, cc) && seg_table(a, 1, cu) && seg_table(a, 2, cd);
       for (double **dst : {&coef_ccd[a], &coef_up[a], &coef_dn[a]})
         SCIHPC_HIP(hipMalloc(reinterpret_cast<void **>(dst), sizeof(double) * 12 * n));
       SCIHPC_HIP(hipMemcpyAsync(coef_ccd[a], cc.data(), sizeof(double) * 12 * n, hipMemcpyHostToDevice, stream));
@@ -1680,8 +2078,105 @@ struct scihpc_ls {
     SCIHPC_HIP(hipHostMalloc(reinterpret_cast<void **>(&lhost), sizeof(double) * 2 * nb, hipHostMallocDefault));
   }
 
+  // k_twin_seg's table of one line system: the rows of the factorised
+  // coefficients cf (12 n) up to where they repeat, one period, and the last
+  // row; false when they do not repeat soon enough
+  bool seg_table(int a, int kind, const std::vector<double> &cf) {
+#pragma clang fp contract(off)
+    const int n = g.N[a];
+    auto same = [&](int i, int j) {
+      for (int e = 0; e < 12; ++e)
+        if (std::memcmp(&cf[(size_t)e * n + i], &cf[(size_t)e * n + j], sizeof(double)) != 0) return false;
+      return true;
+    };
+    // rows 0 .. n - 2 repeat with `period` from `start` on (short lines: all rows are kept)
+    int start = n - 1, period = 1;
+    if (n > kTwinRowsMax) {
+      bool found = false;
+      for (int p = 1; p <= 6 && !found; ++p) {  // divisors of k_twin_seg's block of six steps
+        if (6 % p != 0) continue;
+        int i = n - 2 - p;
+        while (i >= 0 && same(i, i + p)) --i;
+        if (i + 1 + p + 1 <= kTwinRowsMax) {
+          start = i + 1;
+          period = p;
+          found = true;
+        }
+      }
+      if (!found) return false;
+    }
+    const int rows = std::min(n - 1, start + (n - 1 > start ? period : 0)) + 1;
+    std::vector<double> t((size_t)kTwinRow * rows);
+    for (int r = 0; r < rows; ++r) {
+      const int i = r == rows - 1 ? n - 1 : r;
+      auto c = [&](int e, int band) { return cf[(size_t)(3 * e + band) * n + i]; };
+      double *o = &t[(size_t)kTwinRow * r];
+      for (int e = 0; e < 4; ++e) {
+        o[e] = c(e, 0);
+        o[4 + e] = c(e, 2);
+        o[8 + e] = c(e, 1);
+      }
+      o[12] = o[8] * o[11] - o[10] * o[9];
+      o[13] = 1.0 / o[12];
+    }
+    SCIHPC_HIP(hipMalloc(reinterpret_cast<void **>(&seg_rows[a][kind]), sizeof(double) * t.size()));
+    SCIHPC_HIP(hipMemcpyAsync(seg_rows[a][kind], t.data(), sizeof(double) * t.size(), hipMemcpyHostToDevice, stream));
+    SCIHPC_HIP(hipStreamSynchronize(stream));
+    seg_start[a][kind] = start;
+    seg_period[a][kind] = period;
+    seg_count[a][kind] = rows;
+    return true;
+  }
+
+  // the segmented sweeps over lines that fit LDS; false when they do not
+  template <int LINES, bool UP>
+  bool twin_seg(const double *f, double *d1[3], double *d2[3]) {
+    constexpr int NS = UP ? 2 : 1;
+    int nmax = 0;
+    for (int a = 0; a < g.ndim; ++a) nmax = std::max(nmax, g.N[a]);
+    TwinPlan pl{};
+    pl.cap = (nmax * LINES + 1) / 2 * 2;
+    const size_t lds = sizeof(double) * ((UP ? 4 : 3) * (size_t)pl.cap + NS * kTwinRow * kTwinRowsMax);
+    if (lds + 1024 > (size_t)lds_max) return false;
+    // about 33 positions a segment on the longest lines
+    pl.waves = std::max(1, std::min(4, (int)std::lround(nmax * LINES / (64.0 * 33.0))));
+    TwinTable tb{};
+    long total = 0;
+    for (int a = 0; a < g.ndim; ++a) {
+      const int n = g.N[a], most = 64 * pl.waves / LINES;
+      pl.len[a] = std::max((n + most - 1) / most, std::min(n, 25)) | 1;
+      pl.segs[a] = (n + pl.len[a] - 1) / pl.len[a];
+      pl.blocks[a] = (int)ceil_div((long)g.N[(a + 1) % 3] * g.N[(a + 2) % 3], LINES);
+      total += pl.blocks[a];
+      for (int y = 0; y < NS; ++y) {
+        const int kind = UP ? 1 + y : 0;
+        tb.row[a][y] = seg_rows[a][kind];
+        tb.start[a][y] = seg_start[a][kind];
+        tb.period[a][y] = seg_period[a][kind];
+        tb.rows[a][y] = seg_count[a][kind];
+      }
+    }
+    if (total > 0x7fffffffL) return false;
+    if (lds > 65536 && !seg_lds_set[UP][LINES / 2]) {
+      SCIHPC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_twin_seg<LINES, UP>),
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
+      seg_lds_set[UP][LINES / 2] = true;
+    }
+    double *none[3] = {nullptr, nullptr, nullptr};
+    double **dd = d2 ? d2 : none;
+    k_twin_seg<LINES, UP><<<(unsigned)total, 64 * NS * pl.waves, lds, stream>>>(g, f, u, v, w, tb, pl, d1[0], d1[1],
+                                                                                d1[2], dd[0], dd[1], dd[2]);
+    SCIHPC_CHECK_LAUNCH();
+    return true;
+  }
+
   // derivatives of f along every real axis: UCCD by (u, v, w) or CCD
   void compact(const double *f, bool upwind, double *d1[3], double *d2[3]) {
+    if (seg_ok && !(twin_lines && twin_partitioned)) {
+      if (upwind ? twin_seg<4, true>(f, d1, d2) || twin_seg<2, true>(f, d1, d2) || twin_seg<1, true>(f, d1, d2)
+                 : twin_seg<4, false>(f, d1, d2) || twin_seg<2, false>(f, d1, d2) || twin_seg<1, false>(f, d1, d2))
+        return;
+    }
     LineScratch sc{};
     LineCoefs co{};
     long work = 0;
@@ -1911,7 +2406,8 @@ extern "C" int scihpc_ls_destroy(scihpc_ls *h) {
                     h->fyy, h->fzz, h->sgn, h->dlt, h->grd, h->flux, h->lpart})
     if (p) (void)hipFree(p);
   for (int a = 0; a < 3; ++a)
-    for (double *p : {h->coef_ccd[a], h->coef_up[a], h->coef_dn[a]})
+    for (double *p : {h->coef_ccd[a], h->coef_up[a], h->coef_dn[a], h->seg_rows[a][0], h->seg_rows[a][1],
+                      h->seg_rows[a][2]})
       if (p) (void)hipFree(p);
   if (h->carry) (void)hipFree(h->carry);
   for (auto &axis : h->ls_scr)
