@@ -7,11 +7,12 @@
 //
 // Storage: the reference's padded scalar_data layout made contiguous
 // (data[i][j][k], k fastest, 3 ghost cells on every axis < ndim).  One
-// fused kernel per RK stage computes the WENO-Z face value on the upwind
-// side only, the convection RHS and the stage update into a second
-// buffer; one small kernel per axis then fills that buffer's ghosts in the
-// reference's order (x, y, z; right side before left side).  Corner ghosts
-// are never written, as in the reference.
+// fused kernel per RK stage computes the WENO-Z face values on the upwind
+// side only, the convection RHS, the stage update into a second buffer and
+// that buffer's ghosts (the reference's order of axes matters only for
+// Dirichlet sides, whose ghosts small kernels per axis fill: x, y, z; right
+// side before left side).  Corner ghosts are never written, as in the
+// reference.
 #include <algorithm>
 #include <cmath>
 #include <cstring>
@@ -131,34 +132,20 @@ __global__ void __launch_bounds__(kLsBlock) k_weno_derivs(Grid g, const double *
   if constexpr (DIM > 2) fz[c] = weno_deriv(f, w, c, g.s[2], g.h[2]);
 }
 
-// One TVD-RK3 stage fused with the convection RHS (source.cpp:12-39):
-// s = -u*fx - v*fy - w*fz on interior cells, then
+// One TVD-RK3 stage of a 1-D field fused with the convection RHS
+// (source.cpp:12-39): s = -u*fx on interior cells, then
 //   stage 1: out = in + dt*s                 (s1 <- s)
 //   stage 2: out = in + dt*(s - 3 s1)/4      (s2 <- s)
 //   stage 3: out = in + dt*(-s1 - s2 + 8 s)/12
-// fx/fy/fz are also stored, as scalar_data keeps them.
-template <int DIM, int STAGE>
+// (2-D and 3-D: k_rk3_fused)
+template <int STAGE>
 __global__ void __launch_bounds__(kLsBlock) k_rk3_stage(Grid g, const double *__restrict__ in, double *__restrict__ out,
-                                                        const double *__restrict__ u, const double *__restrict__ v,
-                                                        const double *__restrict__ w, double *__restrict__ s1,
-                                                        double *__restrict__ s2, double *fx, double *fy, double *fz,
-                                                        double dt) {
+                                                        const double *__restrict__ u, double *__restrict__ s1,
+                                                        double *__restrict__ s2, double dt) {
   const long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (t >= g.interior) return;
   const long c = interior_index(g, t);
-  const double dfx = weno_deriv(in, u, c, g.s[0], g.h[0]);
-  double s = -u[c] * dfx;
-  fx[c] = dfx;
-  if constexpr (DIM > 1) {
-    const double dfy = weno_deriv(in, v, c, g.s[1], g.h[1]);
-    s -= v[c] * dfy;
-    fy[c] = dfy;
-  }
-  if constexpr (DIM > 2) {
-    const double dfz = weno_deriv(in, w, c, g.s[2], g.h[2]);
-    s -= w[c] * dfz;
-    fz[c] = dfz;
-  }
+  const double s = -u[c] * weno_deriv(in, u, c, g.s[0], g.h[0]);
   const double x = in[c];
   if constexpr (STAGE == 1) {
     s1[c] = s;
@@ -294,6 +281,162 @@ __global__ void __launch_bounds__(kLsBlock) k_bc_axis_fields(Grid g, BcFields m,
   const BcSpec &bc = m.bc[q];
   bc_line(p, g.s[a], g.n[a], g.N[a], bc.type[2 * a + 1], true, face, bc.value[2 * a + 1], g.h[a]);
   bc_line(p, g.s[a], g.n[a], g.N[a], bc.type[2 * a], false, face, bc.value[2 * a], g.h[a]);
+}
+
+// ---- fused TVD-RK3 stage, 2-D and 3-D
+// k_rk3_stage<1>'s work with every face value formed once and the ghosts
+// filled by the cells they copy.  The last axis is contiguous: a wavefront
+// takes 64 faces and so 63 cells of a row, each lane handing its face to the
+// next.  Threads march `run` cells along the first axis and carry the face
+// between them.  In 3-D a workgroup is kRkRows rows of the middle axis, the
+// lowest of which only forms faces for the row above it.
+// What bounds it: FP64 issue.  A face took ten IEEE divisions (about 14
+// instructions each) and was formed by both its cells; here it takes four
+// reciprocals (v_rcp_f64 and two Newton steps).  The WENO-Z weights are
+// ratios, so their common denominator is left out and one division by the
+// weights' sum remains, its quotient corrected by its remainder.
+// Measured at 1024 x 512: a stage with its boundary conditions 20.3 + 2 x 4.7
+// us in three launches before, 11.9 us here (a step 81 -> 36 us).
+constexpr int kRkRows = 8;
+
+__device__ __forceinline__ double weno_rcp(double d) {
+  double r = __builtin_amdgcn_rcp(d);
+  r = __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+  return __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
+}
+
+// weno_face(a, b, c, d, e, left-biased): the value right of c
+__device__ __forceinline__ double weno_face_left(double a, double b, double c, double d, double e) {
+  const double p0 = a - 2.0 * b + c, q0 = a - 4.0 * b + 3.0 * c;
+  const double p1 = b - 2.0 * c + d, q1 = b - d;
+  const double p2 = c - 2.0 * d + e, q2 = 3.0 * c - 4.0 * d + e;
+  const double b0 = 13.0 * p0 * p0 + 3.0 * q0 * q0;
+  const double b1 = 13.0 * p1 * p1 + 3.0 * q1 * q1;
+  const double b2 = 13.0 * p2 * p2 + 3.0 * q2 * q2;
+  const double eps = 1e-8;
+  const double tau = fabs(b0 - b2);
+  const double a0 = 1.0 + tau * weno_rcp(eps + b0);
+  const double a1 = 6.0 + 6.0 * tau * weno_rcp(eps + b1);
+  const double a2 = 3.0 + 3.0 * tau * weno_rcp(eps + b2);
+  const double num = a0 * (2.0 * a - 7.0 * b + 11.0 * c) + a1 * (5.0 * c - b + 2.0 * d) + a2 * (2.0 * c + 5.0 * d - e);
+  const double den = 6.0 * (a0 + a1 + a2);
+  const double r = weno_rcp(den), q = num * r;
+  return __builtin_fma(__builtin_fma(-den, q, num), r, q);
+}
+
+// upwinded value right of f[2] from f[0..5]; vel: the two cells' velocities
+__device__ __forceinline__ double weno_upwind(const double (&f)[6], double vl, double vr) {
+  const bool left = vl + vr > 0.0;
+  return weno_face_left(left ? f[0] : f[5], left ? f[1] : f[4], left ? f[2] : f[3], left ? f[3] : f[2],
+                        left ? f[4] : f[1]);
+}
+
+// The ghosts of axis a that a cell-centred BC (but Dirichlet, which changes
+// the boundary cell itself) takes from interior cell i with value x; f: that
+// cell.  bc_line's values, in its order of operations.
+__device__ __forceinline__ void ghosts_of(const BcSpec &bc, int a, int n, double h, long st, int i, double x,
+                                          double *f) {
+  if (i >= kGhc && i < n - kGhc) return;
+  const int l = bc.type[2 * a], r = bc.type[2 * a + 1];
+  if (r == SCIHPC_BC_NEUMANN) {
+    if (i == n - 1) {
+      const double d = bc.value[2 * a + 1] * h;
+      double y = x;
+      for (int q = 1; q <= kGhc; ++q) f[q * st] = y = y + d;
+    }
+  } else if (r == SCIHPC_BC_PERIODIC) {
+    if (i < kGhc) f[(long)n * st] = x;
+  } else if (n - 1 - i < kGhc) {  // no slip, slip
+    f[(long)(2 * (n - 1 - i) + 1) * st] = r == SCIHPC_BC_NO_SLIP ? -x : x;
+  }
+  if (l == SCIHPC_BC_NEUMANN) {
+    if (i == 0) {
+      const double d = bc.value[2 * a] * h;
+      double y = x;
+      for (int q = 1; q <= kGhc; ++q) f[-q * st] = y = y - d;
+    }
+  } else if (l == SCIHPC_BC_PERIODIC) {
+    if (i >= n - kGhc) f[-(long)n * st] = x;
+  } else if (i < kGhc) {
+    f[-(long)(2 * i + 1) * st] = l == SCIHPC_BC_NO_SLIP ? -x : x;
+  }
+}
+
+template <int DIM, int STAGE>
+__global__ void __launch_bounds__(DIM == 3 ? kWave *kRkRows : kLsBlock)
+    k_rk3_fused(Grid g, const double *__restrict__ in, double *__restrict__ out, const double *__restrict__ u,
+                const double *__restrict__ v, const double *__restrict__ w, double *__restrict__ s1,
+                double *__restrict__ s2, double dt, BcSpec bc, int ghosts, int tiles_c, int tiles_r,
+                int run) {
+  constexpr int C = DIM - 1;  // the contiguous axis
+  __shared__ double yf[DIM == 3 ? 2 : 1][DIM == 3 ? kRkRows : 1][kWave];
+  const int lane = (int)threadIdx.x % kWave, row = (int)threadIdx.x / kWave;
+  // 2-D: every wavefront has a tile of its own
+  int tile = DIM == 3 ? (int)blockIdx.x : (int)blockIdx.x * (kLsBlock / kWave) + row;
+  const int tc = tile % tiles_c;
+  tile /= tiles_c;
+  const int tr = DIM == 3 ? tile % tiles_r : 0;
+  if (DIM == 3) tile /= tiles_r;
+  const int i0 = tile * run, i1 = min(g.n[0], i0 + run);
+  if (DIM == 2 && i0 >= g.n[0]) return;  // whole wavefronts, no barrier in 2-D
+  const int nc = g.n[C], nr = DIM == 3 ? g.n[1] : 1;
+  const int c = tc * (kWave - 1) + lane - 1, r = DIM == 3 ? tr * (kRkRows - 1) + row - 1 : 0;
+  const bool own = lane > 0 && c < nc && (DIM == 2 || (row > 0 && r < nr));  // lane 0 and row 0 form faces only
+  const int cc = min(c, nc - 1), rc = min(r, nr - 1);
+  const long sx = g.s[0], sr = g.s[1];
+  const double *vc = DIM == 3 ? w : v;
+  long p = (long)(i0 + g.off[0]) * sx + (DIM == 3 ? (long)(rc + g.off[1]) * sr : 0) + cc + g.off[C];
+  double f[6], uc = u[p];  // f[2]: the cell at hand, along the march
+#pragma unroll
+  for (int q = 0; q < 6; ++q) f[q] = in[p + (q - 3) * sx];
+  double lower = weno_upwind(f, u[p - sx], uc);
+#pragma unroll
+  for (int q = 0; q < 5; ++q) f[q] = f[q + 1];
+  for (int i = i0; i < i1; ++i, p += sx) {
+    f[5] = in[p + 3 * sx];
+    double a[6];
+#pragma unroll
+    for (int q = 0; q < 6; ++q) a[q] = q == 2 ? f[2] : in[p + q - 2];
+    const double vl = vc[p], ur = u[p + sx];
+    const double fc = weno_upwind(a, vl, vc[p + 1]);
+    const double upper = weno_upwind(f, uc, ur);
+    double fr = 0.0, vr = 0.0;
+    if constexpr (DIM == 3) {
+#pragma unroll
+      for (int q = 0; q < 6; ++q) a[q] = q == 2 ? f[2] : in[p + (q - 2) * sr];
+      vr = v[p];
+      fr = weno_upwind(a, vr, v[p + sr]);
+      yf[i & 1][row][lane] = fr;
+      __syncthreads();
+    }
+    const double fl = __shfl_up(fc, 1, kWave);
+    if (own) {
+      double s = -uc * ((upper - lower) / g.h[0]);
+      if constexpr (DIM == 3) s -= vr * ((fr - yf[i & 1][row - 1][lane]) / g.h[1]);
+      s -= vl * ((fc - fl) / g.h[C]);
+      const double x = f[2];
+      double y;
+      if constexpr (STAGE == 1) {
+        s1[p] = s;
+        y = x + dt * s;
+      } else if constexpr (STAGE == 2) {
+        s2[p] = s;
+        y = x + dt * (s - 3.0 * s1[p]) / 4.0;
+      } else {
+        y = x + dt * (-s1[p] - s2[p] + 8.0 * s) / 12.0;
+      }
+      out[p] = y;
+      if (ghosts) {
+        ghosts_of(bc, 0, g.n[0], g.h[0], sx, i, y, out + p);
+        if constexpr (DIM == 3) ghosts_of(bc, 1, nr, g.h[1], sr, r, y, out + p);
+        ghosts_of(bc, C, nc, g.h[C], 1, c, y, out + p);
+      }
+    }
+    lower = upper;
+    uc = ur;
+#pragma unroll
+    for (int q = 0; q < 5; ++q) f[q] = f[q + 1];
+  }
 }
 
 // find_density: rho = H + (1-H) ratio (or mirrored), lsm.cpp:8-18
@@ -2320,23 +2463,46 @@ struct scihpc_ls {
 #undef SCIHPC_REDIST
   }
 
+  // one WENO stage with its boundary conditions: in the stage's kernel but
+  // for Dirichlet sides, which change boundary cells other axes read
+  template <int DIM, int STAGE>
+  void rk3_stage(const double *in, double *out, double dt) {
+    if constexpr (DIM == 1) {
+      k_rk3_stage<STAGE><<<grid_interior(), kLsBlock, 0, stream>>>(g, in, out, u, s1, s2, dt);
+      SCIHPC_CHECK_LAUNCH();
+      apply_bc(out, -1);
+    } else {
+      bool dirichlet = false;
+      for (int q = 0; q < 2 * DIM; ++q) dirichlet = dirichlet || bc.type[q] == SCIHPC_BC_DIRICHLET;
+      const int tc = (int)ceil_div(g.n[DIM - 1], kWave - 1), tr = DIM == 3 ? (int)ceil_div(g.n[1], kRkRows - 1) : 1;
+      // cells a march: a wavefront forms DIM faces a cell and one more, so
+      // long marches form fewer, but the 1024 SIMDs want two or three
+      // wavefronts each to hide their chains.  Microseconds a step measured with
+      // 1 / 2 / 3 / 4 / 6 / 8 cells: 1024 x 512 42 / 39 / 36 / 39 / 40 / 48,
+      // 333 x 501 21 / 22 / 22 / 24 / 29 / 35, 2048^2 264 / 188 / 163 / 157 /
+      // 145 / 146, 128^3 356 / 273 / 245 / 246 / 224 / 231.
+      int run = 6;
+      auto waves = [&](int q) { return (long)tc * tr * ceil_div(g.n[0], q) * (DIM == 3 ? kRkRows : 1); };
+      while (run > 1 && waves(run) < (DIM == 3 ? 1536 : 2560)) --run;
+      const long tiles = (long)tc * tr * ceil_div(g.n[0], run);
+      constexpr int per = DIM == 3 ? 1 : kLsBlock / kWave;
+      k_rk3_fused<DIM, STAGE><<<ceil_div(tiles, per), DIM == 3 ? kWave * kRkRows : kLsBlock, 0, stream>>>(
+          g, in, out, u, v, w, s1, s2, dt, bc, dirichlet ? 0 : 1, tc, tr, run);
+      SCIHPC_CHECK_LAUNCH();
+      if (dirichlet) apply_bc(out, -1);
+    }
+  }
+
   template <int DIM>
   void rk3_step(double dt) {
     if (scheme == 1) {
       uccd_step<DIM>(dt);
       return;
     }
-    const unsigned nb = grid_interior();
     double *a = phi[cur], *b = phi[cur ^ 1];
-    k_rk3_stage<DIM, 1><<<nb, kLsBlock, 0, stream>>>(g, a, b, u, v, w, s1, s2, fx, fy, fz, dt);
-    SCIHPC_CHECK_LAUNCH();
-    apply_bc(b, -1);
-    k_rk3_stage<DIM, 2><<<nb, kLsBlock, 0, stream>>>(g, b, a, u, v, w, s1, s2, fx, fy, fz, dt);
-    SCIHPC_CHECK_LAUNCH();
-    apply_bc(a, -1);
-    k_rk3_stage<DIM, 3><<<nb, kLsBlock, 0, stream>>>(g, a, b, u, v, w, s1, s2, fx, fy, fz, dt);
-    SCIHPC_CHECK_LAUNCH();
-    apply_bc(b, -1);
+    rk3_stage<DIM, 1>(a, b, dt);
+    rk3_stage<DIM, 2>(b, a, dt);
+    rk3_stage<DIM, 3>(a, b, dt);
     cur ^= 1;
   }
 
