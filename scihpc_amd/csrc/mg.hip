@@ -387,6 +387,7 @@ __global__ void __launch_bounds__(kBlock) k_coarse_solve(DLevel<T> G, const doub
 
 }  // namespace scihpc
 #include "mg_block.hpp"
+#include "mg_tile3d.hpp"
 namespace scihpc {
 
 // ---------------------------------------- fused 2-D fine-level kernels
@@ -2308,7 +2309,42 @@ struct scihpc_mg {
   template <typename T>
   bool z3_level(const std::vector<Level<T>> &lv, int l) const {
     const auto &a = lv[l];
-    return tiled3d && ndim == 3 && a.nx >= 16 && a.ny >= 8 && a.nz >= 8;
+    return tiled3d && ndim == 3 && a.nx >= 16 && a.ny >= 8 && a.nz >= 8 && a.n > kColor3;
+  }
+  // Below this many cells the z-marching sweeps lose to two colour passes: at
+  // 64^3, 32^3 and 16^3 a sweep took 17 to 23 us whatever the size, a colour
+  // pass 3 to 5.
+  static constexpr long kColor3 = 1L << 18;
+  // levels whose whole smoothing is one launch (k_pre3d, k_post3d): factor 2
+  // to the next level, up to 2^18 cells.  At 64^3 the two launches take 15 + 16
+  // us (FP32) and 18 + 20 (FP64), at 32^3 9 + 11 (FP64); the eight colour
+  // passes, restriction and prolongation with their gaps 53 and 50 us.  At
+  // 128^3 they lose: 93 + 96 against about 125 us.
+  template <typename T>
+  bool tile3_level(const std::vector<Level<T>> &lv, int l) const {
+    const auto &a = lv[l];
+    return tiled3d && ndim == 3 && l + 1 < L && lv[l + 1].deg / a.deg == 2 && a.n <= kTile3;
+  }
+  static constexpr long kTile3 = 1L << 18;
+  template <typename T>
+  static unsigned tiles3d(const Level<T> &l) {
+    return (unsigned)((long)ceil_div(l.nx, kT3) * ceil_div(l.ny, kT3) * ceil_div(l.nz, kT3));
+  }
+  template <typename T>
+  void pre3d(std::vector<Level<T>> &lv, int l, int nu1) {
+    auto &a = lv[l];
+    if (variable) k_pre3d<T, true><<<tiles3d(a), kT3Threads, 0, stream>>>(view(a), view(lv[l + 1]), a.sol, nu1);
+    else k_pre3d<T, false><<<tiles3d(a), kT3Threads, 0, stream>>>(view(a), view(lv[l + 1]), a.sol, nu1);
+    SCIHPC_CHECK_LAUNCH();
+  }
+  template <typename T>
+  void post3d(std::vector<Level<T>> &lv, int l, int nu2) {
+    auto &a = lv[l];
+    const int dir = bc == SCIHPC_MG_DIRICHLET;
+    if (variable) k_post3d<T, true><<<tiles3d(a), kT3Threads, 0, stream>>>(view(lv[l + 1]), view(a), a.sol_alt, nu2, dir);
+    else k_post3d<T, false><<<tiles3d(a), kT3Threads, 0, stream>>>(view(lv[l + 1]), view(a), a.sol_alt, nu2, dir);
+    SCIHPC_CHECK_LAUNCH();
+    std::swap(a.sol, a.sol_alt);
   }
   // coefficient source of a level: 2 density (level 0 of A(rho)), 1 faces, 0 constant
   template <typename T>
@@ -2570,12 +2606,15 @@ struct scihpc_mg {
       const int z = (l == 0 && zg) ? 1 : 0;
       if (can_tile && fused_level(lv, l)) {
         pre2d(lv, l, nu1, z);
+      } else if (can_tile && nu1 > 0 && (l > 0 || z) && tile3_level(lv, l)) {
+        pre3d(lv, l, nu1);
       } else if (z3_level(lv, l) && lv[l + 1].deg / lv[l].deg == 2) {
         for (int s = 0; s < nu1; ++s) sweep3(lv, l, 0, s == 0 ? z : 0);
         rr3(lv, l);
       } else {
         for (int s = 0; s < nu1; ++s) sweep(lv[l], 0, s == 0 ? z : 0);
-        residual_restrict(lv[l], lv[l + 1]);
+        if (ndim == 3 && lv[l + 1].deg / lv[l].deg == 2) rr3(lv, l);
+        else residual_restrict(lv[l], lv[l + 1]);
       }
     }
     if (lb < L) {
@@ -2597,6 +2636,8 @@ struct scihpc_mg {
           post0_done = true;
           partials = mode != 0 ? (int)tiles2d(lv[0], 0) : 0;
         }
+      } else if (can_tile && nu2 > 0 && tile3_level(lv, f)) {
+        post3d(lv, f, nu2);
       } else if (z3_level(lv, f)) {
         prolong_add(lv[l], lv[f]);
         for (int s = 0; s < nu2; ++s) sweep3(lv, f, 1, 0);

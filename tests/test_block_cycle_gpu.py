@@ -2,7 +2,7 @@
 go wrong: a single (coarsest) level, odd sizes (a pair with no odd cell),
 ragged patches, factor-3 levels, every patch height, a large coarsest
 matrix, 2-D and 3-D, zero and non-zero initial iterates, unequal sweep
-counts.
+counts; and the 3-D tiles (k_pre3d, k_post3d) above it, whole and ragged.
 
 Bars: FP64 iterates within 1e-10 relative of the oracle's red-black cycle
 (both sum five or seven terms in FP64; the cycles amplify that by far less
@@ -41,7 +41,9 @@ CASES = [
     ((18, 18, 18), "neumann", True),   # 9^3 coarsest
     ((16, 16, 16), "dirichlet", False),
     ((30, 18, 24), "neumann", True),
-    ((32, 32, 32), "neumann", True),
+    ((32, 32, 32), "neumann", True),   # 3-D tiles on level 0 (first cycle only: from zero)
+    ((64, 32, 48), "dirichlet", False),
+    ((72, 60, 48), "neumann", True),   # also on 36 x 30 x 24: ragged in x and y
 ]
 
 
