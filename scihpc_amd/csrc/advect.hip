@@ -617,6 +617,13 @@ struct FlowParams {
 };
 
 __device__ __forceinline__ void padded_ijk(const Grid &g, long c, int q[3]) {
+  if (g.total <= 0xffffffffL) {  // 64-bit divisions cost several times as much
+    const unsigned u = (unsigned)c, w = u / (unsigned)g.s[1];
+    q[0] = (int)(u / (unsigned)g.s[0]);
+    q[1] = (int)(w % (unsigned)g.N[1]);
+    q[2] = (int)(u % (unsigned)g.N[2]);
+    return;
+  }
   q[0] = (int)(c / g.s[0]);
   q[1] = (int)((c / g.s[1]) % g.N[1]);
   q[2] = (int)(c % g.N[2]);
@@ -1859,26 +1866,72 @@ __global__ void __launch_bounds__(kLsBlock)
   if (delta) delta[c] = ls_delta(x, w);
 }
 
-// weno5_for_godunov (godunov_gradient.cpp:184-201)
+// weno5_for_godunov (godunov_gradient.cpp:184-201): w0 / 3 (a - 2b + c) +
+// (w2 - 1/2) / 6 (b - 2c + d) with weights w_k = alpha_k / (alpha_0 +
+// alpha_1 + alpha_2), alpha = (1, 6, 3) / e_k^2.  Over their common
+// denominator the weights are products of the e_k^2, and one reciprocal
+// takes the place of seven IEEE divisions.  Those products leave the range
+// of a double for e beyond 1e50: there the e_k are first divided by the
+// smallest, and one that is still beyond 1e50 weighs less than 1e-100.
 __device__ __forceinline__ double weno_godunov(double a, double b, double c, double d) {
-#pragma clang fp contract(off)
   const double eps = 1e-8;
   const double t0 = a - b, t1 = a - 3.0 * b, t2 = b - c, t3 = b + c, t4 = c - d, t5 = 3.0 * c - d;
-  const double is0 = 13.0 * (t0 * t0) + 3.0 * (t1 * t1);
-  const double is1 = 13.0 * (t2 * t2) + 3.0 * (t3 * t3);
-  const double is2 = 13.0 * (t4 * t4) + 3.0 * (t5 * t5);
-  const double e0 = eps + is0, e1 = eps + is1, e2 = eps + is2;
-  const double alp0 = 1.0 / (e0 * e0), alp1 = 6.0 / (e1 * e1), alp2 = 3.0 / (e2 * e2);
-  const double w0 = alp0 / (alp0 + alp1 + alp2);
-  const double w2 = alp2 / (alp0 + alp1 + alp2);
-  return w0 / 3.0 * (a - 2.0 * b + c) + (w2 - 0.5) / 6.0 * (b - 2.0 * c + d);
+  double e0 = eps + (13.0 * (t0 * t0) + 3.0 * (t1 * t1));
+  double e1 = eps + (13.0 * (t2 * t2) + 3.0 * (t3 * t3));
+  double e2 = eps + (13.0 * (t4 * t4) + 3.0 * (t5 * t5));
+  if (fmax(e0, fmax(e1, e2)) > 1e50) {
+    const double lo = fmin(e0, fmin(e1, e2));
+    e0 = fmin(e0 / lo, 1e50);
+    e1 = fmin(e1 / lo, 1e50);
+    e2 = fmin(e2 / lo, 1e50);
+  }
+  e0 *= e0;
+  e1 *= e1;
+  e2 *= e2;
+  const double p = e1 * e2, q = 6.0 * (e0 * e2), r = 3.0 * (e0 * e1);
+  const double v = weno_rcp(12.0 * (p + q + r));
+  return 4.0 * p * v * (a - 2.0 * b + c) + (r - p - q) * v * (b - 2.0 * c + d);
+}
+
+struct GodunovH {
+  double h12[3], h[3];  // 1 / (12 h) and 1 / h
+};
+static GodunovH godunov_h(const Grid &g) {
+  GodunovH r;
+  for (int a = 0; a < 3; ++a) {
+    r.h12[a] = 1.0 / (12.0 * g.h[a]);
+    r.h[a] = 1.0 / g.h[a];
+  }
+  return r;
+}
+
+// one axis' share of the squared Godunov gradient at phi[0] (stride st; cell
+// size h: rh12 = 1 / (12 h), rh = 1 / h): the upwind one-sided slope, squared
+__device__ __forceinline__ double godunov_axis(const double *__restrict__ phi, long st, double rh12, double rh,
+                                               bool inside) {
+#pragma clang fp contract(off)
+#define P(k) phi[(k) * st]
+  const double v =
+      rh12 * (-(P(-1) - P(-2)) + 7.0 * (P(0) - P(-1)) + 7.0 * (P(1) - P(0)) - (P(2) - P(1)));
+  const double up = v + rh *
+                            weno_godunov(P(3) - 2.0 * P(2) + P(1), P(2) - 2.0 * P(1) + P(0),
+                                         P(1) - 2.0 * P(0) + P(-1), P(0) - 2.0 * P(-1) + P(-2));
+  const double um = v - rh *
+                            weno_godunov(P(-3) - 2.0 * P(-2) + P(-1), P(-2) - 2.0 * P(-1) + P(0),
+                                         P(-1) - 2.0 * P(0) + P(1), P(0) - 2.0 * P(1) + P(2));
+#undef P
+  double m;
+  if (inside) m = fmax(-fmin(up, 0.0), fmax(um, 0.0));
+  else m = fmax(fmax(up, 0.0), -fmin(um, 0.0));
+  return m * m;
 }
 
 // godunov_gradient (godunov_gradient.cpp:7-152) on every padded cell (0 on
 // the ghosts)
 template <int DIM>
 __global__ void __launch_bounds__(kLsBlock)
-    k_godunov(Grid g, const double *__restrict__ phi, const double *__restrict__ sign, double *__restrict__ grad) {
+    k_godunov(Grid g, GodunovH r, const double *__restrict__ phi, const double *__restrict__ sign,
+              double *__restrict__ grad) {
 #pragma clang fp contract(off)
   const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= g.total) return;
@@ -1891,45 +1944,52 @@ __global__ void __launch_bounds__(kLsBlock)
   if (in) {
 #pragma unroll
     for (int a = 0; a < DIM; ++a) {
-      const long s = g.s[a];
-      const double h = g.h[a];
-#define P(k) phi[c + (k) * s]
-      const double v = 1.0 / (12.0 * h) *
-                       (-(P(-1) - P(-2)) + 7.0 * (P(0) - P(-1)) + 7.0 * (P(1) - P(0)) - (P(2) - P(1)));
-      const double up = v + 1.0 / h *
-                                weno_godunov(P(3) - 2.0 * P(2) + P(1), P(2) - 2.0 * P(1) + P(0),
-                                             P(1) - 2.0 * P(0) + P(-1), P(0) - 2.0 * P(-1) + P(-2));
-      const double um = v - 1.0 / h *
-                                weno_godunov(P(-3) - 2.0 * P(-2) + P(-1), P(-2) - 2.0 * P(-1) + P(0),
-                                             P(-1) - 2.0 * P(0) + P(1), P(0) - 2.0 * P(1) + P(2));
-#undef P
-      double m;
-      if (sign[c] > 0.0) m = fmax(-fmin(up, 0.0), fmax(um, 0.0));
-      else m = fmax(fmax(up, 0.0), -fmin(um, 0.0));
-      gsum = a == 0 ? m * m : gsum + m * m;
+      const double m2 = godunov_axis(phi + c, g.s[a], r.h12[a], r.h[a], sign[c] > 0.0);
+      gsum = a == 0 ? m2 : gsum + m2;
     }
   }
   grad[c] = sqrt(gsum);
 }
 
-// lsf_redistance_lambda (source.cpp:148-240) and the RK3 stage update on
-// every padded cell, in place; a and b at the diagonal neighbours are read
-// at clamped positions (zero_order_extrapolation, simple_bc.cpp:7-43)
+// The RK3 stage update of redistancing at padded cell c: from value x and
+// rate s
+template <int STAGE>
+__device__ __forceinline__ double redist_update(double x, double s, long c, double *__restrict__ s1,
+                                                double *__restrict__ s2, double dt) {
+#pragma clang fp contract(off)
+  if (STAGE == 1) {
+    s1[c] = s;
+    return x + dt * s;
+  }
+  if (STAGE == 2) {
+    s2[c] = s;
+    return x + dt * (s - 3.0 * s1[c]) / 4.0;
+  }
+  return x + dt * (-s1[c] - s2[c] + 8.0 * s) / 12.0;
+}
+
+// lsf_redistance_lambda (source.cpp:148-240), the RK3 stage update and the
+// ghosts of any boundary condition but Dirichlet (`ghosts`) in place, 1-D and
+// 3-D; a and b at the diagonal neighbours are read at clamped positions
+// (zero_order_extrapolation, simple_bc.cpp:7-43).  Ghosts outside on one axis
+// are their boundary condition's; those outside on more are advanced like
+// cells of zero gradient.
 template <int DIM, int STAGE>
 __global__ void __launch_bounds__(kLsBlock)
     k_redist_stage(Grid g, double *__restrict__ phi, const double *__restrict__ sign,
                    const double *__restrict__ delta, const double *__restrict__ grad, double *__restrict__ s1,
-                   double *__restrict__ s2, double dt, double rdt) {
+                   double *__restrict__ s2, double dt, double rdt, BcSpec bc, int ghosts) {
 #pragma clang fp contract(off)
   const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= g.total) return;
   int q[3];
   padded_ijk(g, c, q);
-  double s = -sign[c] * (grad[c] - 1.0) * rdt / dt;
-  bool in = true;
+  int out = 0;
 #pragma unroll
-  for (int a = 0; a < DIM; ++a) in = in && q[a] >= g.off[a] && q[a] < g.off[a] + g.n[a];
-  if (in && DIM >= 2) {
+  for (int a = 0; a < DIM; ++a) out += q[a] < g.off[a] || q[a] >= g.off[a] + g.n[a];
+  if (out == 1) return;
+  double s = -sign[c] * (grad[c] - 1.0) * rdt / dt;
+  if (out == 0 && DIM == 3) {
     auto AB = [&](int di, int dj, int dk, double &A, double &B) {
       int r[3] = {q[0] + di, q[1] + dj, q[2] + dk};
       const long p = ext_index<DIM>(g, r, -1);
@@ -1938,37 +1998,77 @@ __global__ void __launch_bounds__(kLsBlock)
     };
     double A, B;
     AB(0, 0, 0, A, B);
-    double a, b;
-    if (DIM == 2) {
-      a = 16.0 * A;
-      b = 16.0 * B;
-      for (int ii = -1; ii < 2; ii += 2)
-        for (int jj = -1; jj < 2; jj += 2) {
-          AB(ii, jj, 0, A, B);
+    double a = 51.0 * A, b = 51.0 * B;
+    for (int ii = -1; ii < 2; ii += 2)
+      for (int jj = -1; jj < 2; jj += 2)
+        for (int kk = -1; kk < 2; kk += 2) {
+          AB(ii, jj, kk, A, B);
           a += A;
           b += B;
         }
-    } else {
-      a = 51.0 * A;
-      b = 51.0 * B;
-      for (int ii = -1; ii < 2; ii += 2)
-        for (int jj = -1; jj < 2; jj += 2)
-          for (int kk = -1; kk < 2; kk += 2) {
-            AB(ii, jj, kk, A, B);
-            a += A;
-            b += B;
-          }
-    }
     if (fabs(b) > 1e-8) s += a / b * delta[c] * grad[c] * rdt / dt;
   }
-  if (STAGE == 1) {
-    s1[c] = s;
-    phi[c] += dt * s;
-  } else if (STAGE == 2) {
-    s2[c] = s;
-    phi[c] += dt * (s - 3.0 * s1[c]) / 4.0;
-  } else {
-    phi[c] += dt * (-s1[c] - s2[c] + 8.0 * s) / 12.0;
+  const double y = redist_update<STAGE>(phi[c], s, c, s1, s2, dt);
+  phi[c] = y;
+  if (out == 0 && ghosts) {
+#pragma unroll
+    for (int a = 0; a < DIM; ++a) ghosts_of(bc, a, g.n[a], g.h[a], g.s[a], q[a] - g.off[a], y, phi + c);
+  }
+}
+
+// k_godunov and k_redist_stage in one launch for 2-D, from `in` to `outp`.
+// A thread forms the gradient of one position of a 16 x 32 tile, clamped to
+// the interior; a and b stay in LDS for the diagonal neighbours, and the
+// inner 14 x 30 positions are advanced.  The rim's gradients are formed twice
+// (512 for 420 cells), which costs less than the gradient's way through
+// memory and a launch.  What bounds it: FP64 issue, some 480 instructions a
+// position, and on small grids the chain of one wavefront.
+// Measured: a step's three stages at 501 x 333 65 us in twelve launches
+// before, 24 here; 64 x 128 16 us, 1024^2 74, 3000 x 2000 368.  Tiles of 8 x
+// 32 / 8 x 64 / 16 x 16: 25 / 24 / 26, 15 / 17 / 15, 79 / 78 / 77, 390 / 401
+// / 378 us.
+constexpr int kRdRows = 16, kRdCols = 32;
+template <int STAGE>
+__global__ void __launch_bounds__(kRdRows *kRdCols)
+    k_redist2d(Grid g, GodunovH r, const double *__restrict__ in, double *__restrict__ outp, const double *__restrict__ sign,
+               const double *__restrict__ delta, double *__restrict__ s1, double *__restrict__ s2, double dt,
+               double rdt, BcSpec bc, int ghosts, int tiles_c) {
+#pragma clang fp contract(off)
+  __shared__ double As[kRdRows][kRdCols], Bs[kRdRows][kRdCols];
+  const int ty = (int)threadIdx.x / kRdCols, tx = (int)threadIdx.x % kRdCols;
+  const int tr = (int)blockIdx.x / tiles_c, tc = (int)blockIdx.x - tr * tiles_c;
+  const int i = tr * (kRdRows - 2) + ty - 1, j = tc * (kRdCols - 2) + tx - 1;  // padded
+  const int ci = clampi(i, g.off[0], g.off[0] + g.n[0] - 1), cj = clampi(j, g.off[1], g.off[1] + g.n[1] - 1);
+  const long c = (long)ci * g.s[0] + (long)cj * g.s[1];
+  const double sg = sign[c], dl = delta[c], x = in[c];
+  double gr = godunov_axis(in + c, g.s[0], r.h12[0], r.h[0], sg > 0.0);
+  gr = sqrt(gr + godunov_axis(in + c, g.s[1], r.h12[1], r.h[1], sg > 0.0));
+  const double A = sg * dl * (gr - 1.0), B = gr * dl * dl;
+  As[ty][tx] = A;
+  Bs[ty][tx] = B;
+  __syncthreads();
+  const bool own = ty > 0 && ty < kRdRows - 1 && tx > 0 && tx < kRdCols - 1 && i < g.N[0] && j < g.N[1];
+  if (!own || (i != ci) != (j != cj)) return;
+  if (i != ci) {  // a corner's ghost: gradient 0
+    const long p = (long)i * g.s[0] + (long)j * g.s[1];
+    outp[p] = redist_update<STAGE>(in[p], -sign[p] * (0.0 - 1.0) * rdt / dt, p, s1, s2, dt);
+    return;
+  }
+  double s = -sg * (gr - 1.0) * rdt / dt;
+  double a = 16.0 * A, b = 16.0 * B;
+#pragma unroll
+  for (int ii = -1; ii < 2; ii += 2)
+#pragma unroll
+    for (int jj = -1; jj < 2; jj += 2) {
+      a += As[ty + ii][tx + jj];
+      b += Bs[ty + ii][tx + jj];
+    }
+  if (fabs(b) > 1e-8) s += a / b * dl * gr * rdt / dt;
+  const double y = redist_update<STAGE>(x, s, c, s1, s2, dt);
+  outp[c] = y;
+  if (ghosts) {
+    ghosts_of(bc, 0, g.n[0], g.h[0], g.s[0], i - g.off[0], y, outp + c);
+    ghosts_of(bc, 1, g.n[1], g.h[1], g.s[1], j - g.off[1], y, outp + c);
   }
 }
 
@@ -2446,21 +2546,40 @@ struct scihpc_ls {
     apply_bc(f, -1);
   }
 
-  // tvd_rk3 with lsf_redistance_lambda on the stored sign and delta
+  // boundary conditions of phi that change boundary cells, which other
+  // axes read: they can't be filled by the cells they copy
+  bool dirichlet() const {
+    for (int q = 0; q < 2 * g.ndim; ++q)
+      if (bc.type[q] == SCIHPC_BC_DIRICHLET) return true;
+    return false;
+  }
+
+  // one stage of redistancing with its boundary conditions
+  template <int DIM, int STAGE>
+  void redist_stage(const double *in, double *out, double dt, double rdt) {
+    const bool d = dirichlet();
+    if constexpr (DIM == 2) {
+      const unsigned tc = ceil_div(g.N[1], kRdCols - 2), tr = ceil_div(g.N[0], kRdRows - 2);
+      k_redist2d<STAGE><<<tc * tr, kRdRows * kRdCols, 0, stream>>>(g, godunov_h(g), in, out, sgn, dlt, s1, s2, dt, rdt, bc, !d,
+                                                                   (int)tc);
+    } else {
+      const unsigned nb = ceil_div(g.total, kLsBlock);
+      k_godunov<DIM><<<nb, kLsBlock, 0, stream>>>(g, godunov_h(g), out, sgn, grd);
+      SCIHPC_CHECK_LAUNCH();
+      k_redist_stage<DIM, STAGE><<<nb, kLsBlock, 0, stream>>>(g, out, sgn, dlt, grd, s1, s2, dt, rdt, bc, !d);
+    }
+    SCIHPC_CHECK_LAUNCH();
+    if (d) apply_bc(out, -1);
+  }
+
+  // tvd_rk3 with lsf_redistance_lambda on the stored sign and delta; 2-D
+  // stages go from buffer to buffer and end in phi[cur] again
   template <int DIM>
   void redistance_step(double dt, double rdt) {
-    double *f = phi[cur];
-    const unsigned nb = ceil_div(g.total, kLsBlock);
-#define SCIHPC_REDIST(ST)                                                                                  \
-  k_godunov<DIM><<<nb, kLsBlock, 0, stream>>>(g, f, sgn, grd);                                           \
-  SCIHPC_CHECK_LAUNCH();                                                                                   \
-  k_redist_stage<DIM, ST><<<nb, kLsBlock, 0, stream>>>(g, f, sgn, dlt, grd, s1, s2, dt, rdt);            \
-  SCIHPC_CHECK_LAUNCH();                                                                                   \
-  apply_bc(f, -1)
-    SCIHPC_REDIST(1);
-    SCIHPC_REDIST(2);
-    SCIHPC_REDIST(3);
-#undef SCIHPC_REDIST
+    double *f = phi[cur], *a = DIM == 2 ? grd : f, *b = DIM == 2 ? flux : f;
+    redist_stage<DIM, 1>(f, a, dt, rdt);
+    redist_stage<DIM, 2>(a, b, dt, rdt);
+    redist_stage<DIM, 3>(b, f, dt, rdt);
   }
 
   // one WENO stage with its boundary conditions: in the stage's kernel but
@@ -2472,8 +2591,7 @@ struct scihpc_ls {
       SCIHPC_CHECK_LAUNCH();
       apply_bc(out, -1);
     } else {
-      bool dirichlet = false;
-      for (int q = 0; q < 2 * DIM; ++q) dirichlet = dirichlet || bc.type[q] == SCIHPC_BC_DIRICHLET;
+      const bool dir = dirichlet();
       const int tc = (int)ceil_div(g.n[DIM - 1], kWave - 1), tr = DIM == 3 ? (int)ceil_div(g.n[1], kRkRows - 1) : 1;
       // cells a march: a wavefront forms DIM faces a cell and one more, so
       // long marches form fewer, but the 1024 SIMDs want two or three
@@ -2487,9 +2605,9 @@ struct scihpc_ls {
       const long tiles = (long)tc * tr * ceil_div(g.n[0], run);
       constexpr int per = DIM == 3 ? 1 : kLsBlock / kWave;
       k_rk3_fused<DIM, STAGE><<<ceil_div(tiles, per), DIM == 3 ? kWave * kRkRows : kLsBlock, 0, stream>>>(
-          g, in, out, u, v, w, s1, s2, dt, bc, dirichlet ? 0 : 1, tc, tr, run);
+          g, in, out, u, v, w, s1, s2, dt, bc, dir ? 0 : 1, tc, tr, run);
       SCIHPC_CHECK_LAUNCH();
-      if (dirichlet) apply_bc(out, -1);
+      if (dir) apply_bc(out, -1);
     }
   }
 
@@ -2798,9 +2916,10 @@ extern "C" int scihpc_ls_stabilize_gradient(scihpc_ls *h, double *grad, double *
     const long n = h->g.total;
     const unsigned nb = std::min<unsigned>(ceil_div(n, kLsBlock), 1024);
     double *f = h->phi[h->cur];
-    if (h->g.ndim == 1) k_godunov<1><<<ceil_div(n, kLsBlock), kLsBlock, 0, h->stream>>>(h->g, f, h->sgn, h->grd);
-    else if (h->g.ndim == 2) k_godunov<2><<<ceil_div(n, kLsBlock), kLsBlock, 0, h->stream>>>(h->g, f, h->sgn, h->grd);
-    else k_godunov<3><<<ceil_div(n, kLsBlock), kLsBlock, 0, h->stream>>>(h->g, f, h->sgn, h->grd);
+    const GodunovH r = godunov_h(h->g);
+    if (h->g.ndim == 1) k_godunov<1><<<ceil_div(n, kLsBlock), kLsBlock, 0, h->stream>>>(h->g, r, f, h->sgn, h->grd);
+    else if (h->g.ndim == 2) k_godunov<2><<<ceil_div(n, kLsBlock), kLsBlock, 0, h->stream>>>(h->g, r, f, h->sgn, h->grd);
+    else k_godunov<3><<<ceil_div(n, kLsBlock), kLsBlock, 0, h->stream>>>(h->g, r, f, h->sgn, h->grd);
     SCIHPC_CHECK_LAUNCH();
     // maxima into the stage scratch s1: nb block maxima, then one
     k_block_max<<<nb, kLsBlock, 0, h->stream>>>(h->grd, n, h->s1);
