@@ -52,3 +52,29 @@ def test_fused_stage_matches_oracle(oracle, n, bc):
     for a in range(ndim):  # every line through the interior, its ghosts included
         at = tuple(slice(None) if d == a else s for d, s in enumerate(inner))
         assert np.abs(got[at] - want[at]).max() < 1e-13 * big
+
+
+@pytest.mark.parametrize("bc", BCS, ids=lambda b: "-".join(x[:3] for x in b[:4]))
+@pytest.mark.parametrize("n", [(3, 4, 1), (33, 63, 1), (40, 1, 1), (6, 7, 5)], ids=lambda n: "x".join(map(str, n)))
+def test_uccd_stage_fills_its_ghosts(oracle, n, bc):
+    """k_uccd_stage's ghosts: the oracle's bits, corners too (next to a
+    Dirichlet side bc_line fills them, whose U h + F the compiler may round
+    once: values of zero there)"""
+    ndim = 1 if n[1] == 1 else 2 if n[2] == 1 else 3
+    h = (1.0 / n[0], 0.8 / n[1], 1.1 / n[2])
+    shp = padded_shape(ndim, *n)
+    rng = np.random.default_rng(sum(n))
+    phi = rng.standard_normal(shp)
+    vel = [rng.standard_normal(shp) for _ in range(3)]
+    vals = np.zeros(6) if "dirichlet" in bc else np.linspace(-0.3, 0.4, 6)
+    dt = 0.05 * min(h[:ndim])
+    print(f"uccd stage {n} {bc}", flush=True)
+    ls = LevelSet(ndim, *n, *h, bc, list(vals))
+    ls.set_phi(phi)
+    ls.set_velocity(*vel)
+    ls.set_scheme("uccd")
+    ls.tvd_rk3(dt, 2)
+    want = phi.ravel().copy()
+    types = np.array([BC_CODES[b] for b in bc], np.int32)
+    oracle.lib.orc_tvd_rk3_uccd(ndim, *n, *h, dt, types, vals, want, *[a.ravel() for a in vel], 2)
+    np.testing.assert_array_equal(ls.phi().ravel(), want)
