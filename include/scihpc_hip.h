@@ -466,8 +466,10 @@ SCIHPC_API int scihpc_ls_set_scheme(scihpc_ls *h, int scheme);
 /* How the CCD/UCCD line systems are solved (the twin back substitution of
  * matrix_solver.cpp:58-83 on the factorised coefficients of twin_dec,
  * :21-56).  partitioned = 0 (the default): the values of the reference's
- * sequential order, bit for bit (lines are swept in segments that start from
- * overlapping warm-ups, each checked against its neighbour's final state).  partitioned = 1: every line cut
+ * sequential order, bit for bit but for the sign of a zero and the rounding
+ * of results below 2^-1042 in magnitude (lines are swept in segments that
+ * start from overlapping warm-ups, each checked against its neighbour's final
+ * state, where that pays).  partitioned = 1: every line cut
  * into segments that sweep in parallel and exchange their incoming states
  * through 2x2 segment propagators, then sweep again from the true states
  * with the reference's arithmetic; the results differ from the sequential
@@ -476,6 +478,11 @@ SCIHPC_API int scihpc_ls_set_scheme(scihpc_ls *h, int scheme);
  * sequentially).  No counterpart in the reference (its solve is always
  * sequential); for callers that trade the reference's bits for speed. */
 SCIHPC_API int scihpc_ls_set_line_solver(scihpc_ls *h, int partitioned);
+/* Of the line sweeps of this handle so far (partitioned = 0): workgroups
+ * launched to sweep their lines in segments, and those of them that had to
+ * leave their lines to a sweep from end to end.  Waits for the handle's
+ * stream.  No counterpart in the reference. */
+SCIHPC_API int scihpc_ls_line_sweeps(scihpc_ls *h, long long *segmented, long long *end_to_end);
 /* uccd_solver::find_derivatives(f, vel) (upwind = 1, the handle's
  * velocity) or ccd_solver::find_derivatives(f) (ccd_solver.cpp:14-142) of
  * a padded host array: first and second derivatives along every axis. */

@@ -393,6 +393,13 @@ class LevelSet:
         code = {"sequential": 0, "partitioned": 1}[solver]
         check(self._lib.scihpc_ls_set_line_solver(self.h, code))
 
+    def line_sweeps(self):
+        """(workgroups that swept their lines in segments, those of them
+        that left their lines to a sweep from end to end) so far."""
+        seg, whole = C.c_longlong(), C.c_longlong()
+        check(self._lib.scihpc_ls_line_sweeps(self.h, C.byref(seg), C.byref(whole)))
+        return seg.value, whole.value
+
     def compact_derivatives(self, f, upwind=True):
         """UCCD (by the handle's velocity) or CCD derivatives of a padded
         field: (fx, fy, fz, fxx, fyy, fzz)."""

@@ -969,14 +969,21 @@ constexpr int kLineChunk = 16;
 struct LineScratch {
   double *su[3], *ssu[3], *sd[3], *ssd[3];
 };
+// A kernel with a gate does nothing unless *flag is `call` (nullptr: no gate)
+struct LineGate {
+  const unsigned *flag;
+  unsigned call;
+  __device__ __forceinline__ bool closed() const { return flag && *flag != call; }
+};
 struct LineCoefs {
   const double *cu[3], *cd[3];
 };
 
 template <bool UP>
 __global__ void __launch_bounds__(kLsBlock)
-    k_compact_rhs(Grid g, const double *__restrict__ f, LineScratch sc) {
+    k_compact_rhs(Grid g, const double *__restrict__ f, LineScratch sc, LineGate gate) {
 #pragma clang fp contract(off)
+  if (gate.closed()) return;
   const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= g.total) return;
   int q[3];
@@ -1004,8 +1011,10 @@ __global__ void __launch_bounds__(kLsBlock)
 
 // twin_bks (matrix_solver.cpp:58-83) in place on S/SS holding the
 // right-hand sides; thread t: axis a, then line t % lines, system t / lines
-__global__ void __launch_bounds__(64) k_twin_line(Grid g, int nsys, LineCoefs co, LineScratch sc) {
+__global__ void __launch_bounds__(64) k_twin_line(Grid g, int nsys, LineCoefs co, LineScratch sc,
+                                                  LineGate gate) {
 #pragma clang fp contract(off)
+  if (gate.closed()) return;
   constexpr int B = kLineChunk;
   long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   int a = 0;
@@ -1104,11 +1113,16 @@ __global__ void __launch_bounds__(64) k_twin_line(Grid g, int nsys, LineCoefs co
 // zero state (or, if that reaches the line's end, from the exact one), sweeps
 // up to its own first position, then sweeps its own positions in place.
 // Whether the incoming state it arrived at equals the neighbour's final value
-// is checked: if all do the result is the sequential sweep's, bit for bit.  If one is not (a chance below 1e-6 a segment with the warm
-// lengths below, measured on random and smooth data; always where the
-// right-hand side is exactly 0 over a whole warm-up), or if a value is not
-// finite or nearly denormal, the workgroup forms its right-hand sides again and
-// sweeps its lines end to end, one thread each, with IEEE quotients.
+// is checked: if all do the result is the sequential sweep's, bit for bit.
+// With the warm lengths below one of the workgroup's 500 states is not equal
+// in 13 of 9.5 million workgroups (random, smooth and distance fields, 300 to
+// 1400 points a line, UCCD; CCD none of 0.25 million), and always where the
+// right-hand side is exactly 0 over a whole warm-up (fields of two values),
+// which a zero state next to another one shows early.  Then, or if a value is
+// not finite or nearly denormal, the workgroup forms its right-hand sides again
+// and sweeps its lines end to end; where there are too many workgroups for that
+// (scihpc_ls::twin_seg) the call is left to the three passes above, which
+// return at once otherwise.
 //
 // A workgroup holds LINES whole lines in LDS, UCCD's two systems side by
 // side, and does everything from the field to the derivatives: right-hand
@@ -1125,11 +1139,12 @@ __global__ void __launch_bounds__(64) k_twin_line(Grid g, int nsys, LineCoefs co
 // banks.
 // What bounds it: the instructions a lone wavefront issues for about 240
 // steps forward and 230 backward (instead of 2 x 1030), and LDS: whole lines
-// leave one workgroup a CU, so 389 workgroups run as two rounds.  Measured at
+// leave one workgroup a CU, so 388 workgroups run as two rounds.  Measured at
 // 1024 x 512: 91 us, where right-hand sides, one thread a line and selection
-// took 11.7 + 383 + 7.2 us in three launches; a UCCD TVD-RK3 step 1.25 ->
-// 0.34 ms.  Lines that do not fit LDS (over about 4700 points) keep the three
-// passes.
+// took 11.7 + 383 + 7.2 us in three launches; a UCCD TVD-RK3 step 1.24 ->
+// 0.30 ms, of a field of two values 1.24 -> 0.77 (end to end with a thread a
+// line and divisions it was 1.24).  Lines that do not fit LDS (over 4416
+// points for UCCD, 6336 for CCD) keep the three passes.
 struct TwinTable {
   const double *row[3][2];           // [axis][system]: rows of kTwinRow values
   int start[3][2], period[3][2], rows[3][2];
@@ -1141,14 +1156,12 @@ struct TwinPlan {
   int len[3], segs[3];               // positions a segment (odd), segments
   int cap;                           // LDS doubles of one array
   int blocks[3];                     // workgroups of each axis
+  unsigned *state;                   // [0]: the last call left to the three passes, [1]: workgroups that failed
+  unsigned call;                     // number of this call
+  int pass_on;                       // a failure leaves the whole call to the three passes
 };
 // warm-up positions [CCD, UCCD upwind, UCCD downwind]
 __device__ constexpr int kTwinWarmF[3] = {102, 210, 48}, kTwinWarmB[3] = {102, 48, 192};
-
-// row of the table for position i
-__device__ __forceinline__ int twin_row(int i, int n, int start, int period, int rows) {
-  return i == n - 1 ? rows - 1 : i < start ? i : start + (i - start) % period;
-}
 
 __device__ __forceinline__ double twin_quot(double a, double d, double r) {
 #pragma clang fp contract(off)
@@ -1157,10 +1170,16 @@ __device__ __forceinline__ double twin_quot(double a, double d, double r) {
   return __builtin_fma(__builtin_fma(-d, q, a), r, q);
 }
 
-// 0 < |x| < 2^-862 (but for the last denormals): there twin_quot's remainders
-// are no longer exact
-__device__ __forceinline__ bool twin_tiny(double x) {
-  return ((unsigned)__double2hiint(x) << 1) - 1u < ((1023u - 862u) << 21) - 1u;
+// 0 < |x| < 2^-862 (but for |x| < 2^-1042): there twin_quot's remainders are
+// no longer exact
+constexpr unsigned kTwinTiny = ((1023u - 862u) << 21) - 1u;
+__device__ __forceinline__ unsigned twin_size(double x) { return ((unsigned)__double2hiint(x) << 1) - 1u; }
+__device__ __forceinline__ bool twin_tiny(double x) { return twin_size(x) < kTwinTiny; }
+
+// the value of the other lane of a pair
+__device__ __forceinline__ double twin_other(double x) {
+  const int lo = __builtin_amdgcn_mov_dpp(__double2loint(x), 0xb1, 0xf, 0xf, true);
+  return __hiloint2double(__builtin_amdgcn_mov_dpp(__double2hiint(x), 0xb1, 0xf, 0xf, true), lo);
 }
 
 template <int LINES, bool UP>
@@ -1172,7 +1191,7 @@ __global__ void __launch_bounds__(512)  // two systems, at most four wavefronts 
 #pragma clang fp contract(off)
   constexpr int NS = UP ? 2 : 1;
   extern __shared__ __align__(16) double twin_lds[];
-  // neighbouring line groups on one XCD: they share the field's cache lines
+  // neighbouring line groups on one XCD, where their number allows: they share the field's cache lines
   int b = blockIdx.x;
   if (gridDim.x % 8 == 0) b = (b % 8) * (int)(gridDim.x / 8) + b / 8;
   int a = 0;
@@ -1182,6 +1201,14 @@ __global__ void __launch_bounds__(512)  // two systems, at most four wavefronts 
   const int tid = threadIdx.x, nt = blockDim.x;
   const int sys = UP ? tid / (64 * pl.waves) : 0;
   const int ts = tid - sys * 64 * pl.waves;
+  __shared__ int whole;  // a thread found that the workgroup's lines have to be swept end to end
+  if (tid == 0) whole = 0;
+  if (pl.pass_on) {  // another workgroup has failed: its lines and these are the three passes' now
+    __shared__ unsigned failed;
+    if (tid == 0) failed = __hip_atomic_load(pl.state, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+    __syncthreads();
+    if (failed == pl.call) return;
+  }
   const int ln = ts % LINES, seg = ts / LINES;
   double *const S = twin_lds + (size_t)sys * 2 * pl.cap, *const SS = S + pl.cap;
   double *const tab = twin_lds + (size_t)(UP ? 4 : 3) * pl.cap;
@@ -1355,41 +1382,23 @@ __global__ void __launch_bounds__(512)  // two systems, at most four wavefronts 
       ph = ph + 1 == period ? 0 : ph + 1;
     }
   };
-  double p = 0.0, q = 0.0, pin, qin;
-  if (on) {
-    const int i = max(lo - kTwinWarmF[kind], 1);
-    if (i == 1 || seg == 0) {
-      p = S[at(0)];
-      q = SS[at(0)];
-    }
-    forward(i, lo, false, p, q);
-  }
-  pin = p;
-  qin = q;
-  __syncthreads();
-  if (on) forward(max(lo, 1), hi, true, p, q);
-  __syncthreads();
-  if (on && seg > 0)
-    bad |= S[at(lo - 1)] != pin || SS[at(lo - 1)] != qin;
   // backward, the same way; the closure at n - 1 is not one of these steps
-  // (kind of quotient: std::true_type IEEE, std::false_type twin_quot).
-  auto solve2 = [&](auto ieee, const double *c, double si, double ti, double &x, double &y) {
-    const double nx = -(c[5] * ti - c[7] * si), ny = c[4] * ti - c[6] * si;
-    x = ieee ? nx / c[8] : twin_quot(nx, c[8], c[9]);
-    y = ieee ? ny / c[8] : twin_quot(ny, c[8], c[9]);
+  auto solve2 = [&](const double *c, double si, double ti, double &x, double &y) {
+    x = twin_quot(-(c[5] * ti - c[7] * si), c[8], c[9]);
+    y = twin_quot(c[4] * ti - c[6] * si, c[8], c[9]);
   };
-  auto brow = [&](auto ieee, const double *c, double vs, double vss, double &x, double &y) {
-    solve2(ieee, c, vs - (c[0] * x + c[1] * y), vss - (c[2] * x + c[3] * y), x, y);
+  auto brow = [&](const double *c, double vs, double vss, double &x, double &y) {
+    solve2(c, vs - (c[0] * x + c[1] * y), vss - (c[2] * x + c[3] * y), x, y);
   };
-  auto bstep = [&](auto ieee, int i, int r, bool keep, double &x, double &y) {
-    brow(ieee, T + r * kTwinRow + 4, S[at(i)], SS[at(i)], x, y);
+  auto bstep = [&](int i, int r, bool keep, double &x, double &y) {
+    brow(T + r * kTwinRow + 4, S[at(i)], SS[at(i)], x, y);
     if (keep) {
       bad |= twin_tiny(x) || twin_tiny(y);
       S[at(i)] = x;
       SS[at(i)] = y;
     }
   };
-  auto backward = [&](auto ieee, int i, int end, bool keep, double &x, double &y) {
+  auto backward = [&](int i, int end, bool keep, double &x, double &y) {
     const int stop = max(end, start);
     if (i >= stop) {
       int ph = (int)((unsigned)(i - start) % (unsigned)period);
@@ -1411,7 +1420,7 @@ __global__ void __launch_bounds__(512)  // two systems, at most four wavefronts 
           }
 #pragma unroll
           for (int k = 0; k < kTwinUnroll; ++k) {
-            brow(ieee, c[k], vs[k], vss[k], x, y);
+            brow(c[k], vs[k], vss[k], x, y);
             if (keep) {
               bad |= twin_tiny(x) || twin_tiny(y);
               S[at(i - k)] = x;
@@ -1422,47 +1431,167 @@ __global__ void __launch_bounds__(512)  // two systems, at most four wavefronts 
         } while (i - kTwinUnroll + 1 >= stop);
       }
       for (; i >= stop; --i) {
-        bstep(ieee, i, start + ph, keep, x, y);
+        bstep(i, start + ph, keep, x, y);
         ph = ph == 0 ? period - 1 : ph - 1;
       }
     }
 #pragma unroll 2
-    for (; i >= end; --i) bstep(ieee, i, i, keep, x, y);
+    for (; i >= end; --i) bstep(i, i, keep, x, y);
   };
-  double x = 0.0, y = 0.0, xin, yin;
+  // A zero state after a warm-up that did not reach the line's start, next to
+  // a segment with another state: the right-hand side is 0 over the whole
+  // warm-up but not before it, and the neighbour's final state is what is left
+  // of that, not 0.  No need to sweep on before the lines are swept end to
+  // end (a pair of segments in two wavefronts is left to the comparison).
+  double p = 0.0, q = 0.0;
+  bool flat = false;
   if (on) {
-    int i = min(hi - 1 + kTwinWarmB[kind], n - 1);
-    if (i == n - 1) {  // the closure
-      solve2(std::false_type(), T + (rows - 1) * kTwinRow + 4, S[at(i)], SS[at(i)], x, y);
-      --i;
-    }
-    backward(std::false_type(), i, hi, false, x, y);
-  }
-  xin = x;
-  yin = y;
-  __syncthreads();
-  if (on) {
-    if (hi == n) {
-      S[at(n - 1)] = x;
-      SS[at(n - 1)] = y;
-    }
-    backward(std::false_type(), min(hi - 1, n - 2), lo, true, x, y);
-    bad |= !(fabs(x) < __builtin_inf()) || !(fabs(y) < __builtin_inf());
-  }
-  __syncthreads();
-  if (on && hi < n)
-    bad |= S[at(hi)] != xin || SS[at(hi)] != yin;
-  if (__syncthreads_or(bad)) {  // one thread a line from end to end
-    fill();
-    __syncthreads();
-    if (seg == 0) {
+    const int i = max(lo - kTwinWarmF[kind], 1);
+    if (i == 1 || seg == 0) {
       p = S[at(0)];
       q = SS[at(0)];
-      forward(1, n, true, p, q);
-      solve2(std::true_type(), T + (rows - 1) * kTwinRow + 4, p, q, x, y);
-      S[at(n - 1)] = x;
-      SS[at(n - 1)] = y;
-      backward(std::true_type(), n - 2, 0, true, x, y);
+    }
+    flat = i > 1;
+    forward(i, lo, false, p, q);
+  }
+  {
+    const int rest = p != 0.0 || q != 0.0, before = __shfl_up(rest, LINES, 64);
+    flat = flat && !rest && before;  // lanes of the first segment keep their own: not flat
+  }
+  // `whole` is written between two barriers and read after the second: a
+  // thread that is ahead can't write it again before all have read it
+  if (flat) whole = 1;
+  __syncthreads();
+  double x = 0.0, y = 0.0;
+  bool alone = whole;
+  if (!alone) {
+    const double pin = p, qin = q;
+    if (on) forward(max(lo, 1), hi, true, p, q);
+    __syncthreads();
+    if (on && seg > 0)
+      bad |= S[at(lo - 1)] != pin || SS[at(lo - 1)] != qin;
+    flat = false;
+    if (on) {
+      int i = min(hi - 1 + kTwinWarmB[kind], n - 1);
+      flat = i < n - 1;
+      if (i == n - 1) {  // the closure
+        solve2(T + (rows - 1) * kTwinRow + 4, S[at(i)], SS[at(i)], x, y);
+        --i;
+      }
+      backward(i, hi, false, x, y);
+    }
+    const int rest = x != 0.0 || y != 0.0, after = __shfl_down(rest, LINES, 64);
+    if (bad || (flat && !rest && after)) whole = 1;
+    __syncthreads();
+    alone = whole;
+  }
+  if (!alone) {
+    const double xin = x, yin = y;
+    if (on) {
+      if (hi == n) {
+        S[at(n - 1)] = x;
+        SS[at(n - 1)] = y;
+      }
+      backward(min(hi - 1, n - 2), lo, true, x, y);
+      bad |= !(fabs(x) < __builtin_inf()) || !(fabs(y) < __builtin_inf());
+    }
+    __syncthreads();
+    if (on && hi < n)
+      bad |= S[at(hi)] != xin || SS[at(hi)] != yin;
+    if (bad) whole = 1;
+    __syncthreads();
+    alone = whole;
+  }
+  if (alone && tid == 0) {
+    atomicAdd(pl.state + 1, 1u);
+    if (pl.pass_on) __hip_atomic_store(pl.state, pl.call, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT);
+  }
+  if (alone && pl.pass_on) return;
+  if (alone) {
+    // From end to end, two lanes a line: one holds f', the other f'', and they
+    // exchange them; a wavefront on its own is bound by the instructions of a
+    // step, and this halves them.  Blocks of steps whose quotients may not be
+    // IEEE ones are done again with divisions.
+    fill();
+    __syncthreads();
+    if (ts < 2 * LINES) {
+      const int half = ts & 1;
+      double *const V = (half ? SS : S) + (ts >> 1);
+      // where this lane's coefficients are in a row: of its own and of the
+      // other's value, in the recurrences (backward: 4 further) and in the
+      // numerators
+      const int cm = half ? 3 : 0, co = half ? 2 : 1, nm = half ? 8 : 11, no = half ? 10 : 9;
+      double m = V[0];
+      auto next = [&](double v, double a, double b) { return v - (a * m + b * twin_other(m)); };
+      auto fone = [&](int i, int r) {
+        m = next(V[i * LINES], T[r * kTwinRow + cm], T[r * kTwinRow + co]);
+        V[i * LINES] = m;
+      };
+      int i = 1;
+      for (; i < min(start, n - 1); ++i) fone(i, i);
+      if (i + kTwinUnroll <= n - 1) {
+        double c[kTwinUnroll][2];
+#pragma unroll
+        for (int k = 0; k < kTwinUnroll; ++k) {
+          const double *r = T + (start + (i - start + k) % period) * kTwinRow;
+          c[k][0] = r[cm];
+          c[k][1] = r[co];
+        }
+        for (; i + kTwinUnroll <= n - 1; i += kTwinUnroll) {
+          double v[kTwinUnroll];
+#pragma unroll
+          for (int k = 0; k < kTwinUnroll; ++k) v[k] = V[(i + k) * LINES];
+#pragma unroll
+          for (int k = 0; k < kTwinUnroll; ++k) V[(i + k) * LINES] = m = next(v[k], c[k][0], c[k][1]);
+        }
+      }
+      for (; i < n - 1; ++i) fone(i, start + (i - start) % period);
+      fone(i, rows - 1);
+      // backward from the closure
+      auto num = [&](double w, double a, double b) { return a * w - b * twin_other(w); };
+      const double *const R = T + (rows - 1) * kTwinRow;
+      V[(n - 1) * LINES] = m = num(m, R[nm], R[no]) / R[12];
+      auto bone = [&](int j, int r) {
+        const double *c = T + r * kTwinRow;
+        V[j * LINES] = m = num(next(V[j * LINES], c[4 + cm], c[4 + co]), c[nm], c[no]) / c[12];
+      };
+      for (i = n - 2; i >= start && (i - start + 1) % kTwinUnroll != 0; --i) bone(i, start + (i - start) % period);
+      if (i >= start) {
+        double c[kTwinUnroll][6];
+#pragma unroll
+        for (int k = 0; k < kTwinUnroll; ++k) {
+          const double *r = T + (start + (kTwinUnroll - 1 - k) % period) * kTwinRow;
+          c[k][0] = r[4 + cm];
+          c[k][1] = r[4 + co];
+          c[k][2] = r[nm];
+          c[k][3] = r[no];
+          c[k][4] = r[12];
+          c[k][5] = r[13];
+        }
+        for (; i >= start; i -= kTwinUnroll) {
+          double v[kTwinUnroll], z[kTwinUnroll];
+#pragma unroll
+          for (int k = 0; k < kTwinUnroll; ++k) v[k] = V[(i - k) * LINES];
+          const double m0 = m;
+          unsigned low = 0xffffffffu;
+#pragma unroll
+          for (int k = 0; k < kTwinUnroll; ++k) {
+            z[k] = m = twin_quot(num(next(v[k], c[k][0], c[k][1]), c[k][2], c[k][3]), c[k][4], c[k][5]);
+            low = min(low, twin_size(m));
+          }
+          int redo = low < kTwinTiny || !(fabs(m) < __builtin_inf());  // what isn't finite stays so
+          redo |= __builtin_amdgcn_mov_dpp(redo, 0xb1, 0xf, 0xf, true);
+          if (redo) {
+            m = m0;
+#pragma unroll
+            for (int k = 0; k < kTwinUnroll; ++k)
+              z[k] = m = num(next(v[k], c[k][0], c[k][1]), c[k][2], c[k][3]) / c[k][4];
+          }
+#pragma unroll
+          for (int k = 0; k < kTwinUnroll; ++k) V[(i - k) * LINES] = z[k];
+        }
+      }
+      for (; i >= 0; --i) bone(i, i);
     }
     __syncthreads();
   }
@@ -1668,8 +1797,9 @@ template <bool UP>
 __global__ void __launch_bounds__(kLsBlock)
     k_compact_select(long total, int ndim, const double *__restrict__ u, const double *__restrict__ v,
                      const double *__restrict__ w, LineScratch sc, double *d1x, double *d1y, double *d1z,
-                     double *d2x, double *d2y, double *d2z) {
+                     double *d2x, double *d2y, double *d2z, LineGate gate) {
 #pragma clang fp contract(off)
+  if (gate.closed()) return;
   const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= total) return;
   const double *vel[3] = {u, v, w};
@@ -2275,8 +2405,12 @@ struct scihpc_ls {
   double *seg_rows[3][3] = {};
   int seg_start[3][3] = {}, seg_period[3][3] = {}, seg_count[3][3] = {};
   bool seg_ok = false;
+  unsigned *seg_state = nullptr;  // TwinPlan::state
+  unsigned seg_call = 0;          // segmented calls so far (never 0 in one)
+  long long seg_groups = 0;       // their workgroups
   bool seg_lds_set[2][3] = {};  // k_twin_seg<LINES, UP> has been allowed its dynamic LDS, [UP][LINES / 2]
   int lds_max = 65536;      // LDS bytes a workgroup may hold on this device
+  int num_cu = 256;         // compute units
   size_t twin_lds_set = 0;  // dynamic LDS the partitioned kernels have been allowed
 
   void ensure_iface() {
@@ -2294,6 +2428,8 @@ struct scihpc_ls {
       SCIHPC_HIP(hipMemcpyAsync(coef_dn[a], cd.data(), sizeof(double) * 12 * n, hipMemcpyHostToDevice, stream));
       SCIHPC_HIP(hipStreamSynchronize(stream));  // the host vectors go out of scope
     }
+    SCIHPC_HIP(hipMalloc(reinterpret_cast<void **>(&seg_state), sizeof(unsigned) * 2));
+    SCIHPC_HIP(hipMemsetAsync(seg_state, 0, sizeof(unsigned) * 2, stream));
     int nmax = 0;
     for (int a = 0; a < g.ndim; ++a) nmax = std::max(nmax, g.N[a]);
     // 16 lines x 64 segments or 8 x 128, segments of 9 (or 17) positions
@@ -2377,16 +2513,17 @@ struct scihpc_ls {
     return true;
   }
 
-  // the segmented sweeps over lines that fit LDS; false when they do not
+  // the segmented sweeps, in the way that pays for these sizes
+  enum SegWay { kSegNoRoom, kSegDone, kSegPassOn, kSegThreePasses };
   template <int LINES, bool UP>
-  bool twin_seg(const double *f, double *d1[3], double *d2[3]) {
+  SegWay twin_seg(const double *f, double *d1[3], double *d2[3]) {
     constexpr int NS = UP ? 2 : 1;
     int nmax = 0;
     for (int a = 0; a < g.ndim; ++a) nmax = std::max(nmax, g.N[a]);
     TwinPlan pl{};
     pl.cap = (nmax * LINES + 1) / 2 * 2;
     const size_t lds = sizeof(double) * ((UP ? 4 : 3) * (size_t)pl.cap + NS * kTwinRow * kTwinRowsMax);
-    if (lds + 1024 > (size_t)lds_max) return false;
+    if (lds + 1024 > (size_t)lds_max) return kSegNoRoom;
     // about 33 positions a segment on the longest lines
     pl.waves = std::max(1, std::min(4, (int)std::lround(nmax * LINES / (64.0 * 33.0))));
     TwinTable tb{};
@@ -2405,7 +2542,30 @@ struct scihpc_ls {
         tb.rows[a][y] = seg_count[a][kind];
       }
     }
-    if (total > 0x7fffffffL) return false;
+    if (total > 0x7fffffffL) return kSegThreePasses;
+    // Segments, or the three passes?  In units of 91 ns a workgroup that has
+    // to sweep its n positions end to end takes 440 + n, the three passes 80 +
+    // 4.1 n of the longest line (latency; many cells take longer).  The line
+    // lies where fields of two values, whose workgroups all fail, take as long
+    // as with the three passes, or where all workgroups run at once.
+    // us a UCCD step, segments (ordinary field / two values) against three
+    // passes: 100^2 132 / 169 : 171, 512^2 305 / 579 : 689, 1024^2 489 / 1329 :
+    // 1377, 1400 x 374 551 / 1259 : 1553, 24^3 79 / 79 : 90; 48^3 251 / 251 :
+    // 172, 96 x 70 x 76 639 / 805 : 321, 900 x 64 x 64 10126 / 11323 : 3511.
+    // Beyond it segments are still tried where ordinary fields gain, but a
+    // failure leaves the call to the three passes: 1400 x 1000 842 / 1855 :
+    // 1681, 2048^2 1575 / 3379 : 3159 (end to end 6668).
+    double work = 0.0;
+    for (int a = 0; a < g.ndim; ++a) work += double(pl.blocks[a]) * (440 + g.N[a]);
+    // workgroups that run side by side: whole lines in LDS, 192 registers a thread
+    const double slots = (double)num_cu * std::max(1, std::min((int)(lds_max / (lds + 1024)), 8 / (NS * pl.waves)));
+    SegWay way = kSegDone;
+    if (total > slots && work / slots > 3.6 * nmax) way = total / slots <= nmax / 220.0 ? kSegPassOn : kSegThreePasses;
+    if (way == kSegThreePasses) return way;
+    pl.state = seg_state;
+    pl.call = ++seg_call;
+    pl.pass_on = way == kSegPassOn;
+    seg_groups += total;
     if (lds > 65536 && !seg_lds_set[UP][LINES / 2]) {
       SCIHPC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_twin_seg<LINES, UP>),
                                      hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
@@ -2416,15 +2576,18 @@ struct scihpc_ls {
     k_twin_seg<LINES, UP><<<(unsigned)total, 64 * NS * pl.waves, lds, stream>>>(g, f, u, v, w, tb, pl, d1[0], d1[1],
                                                                                 d1[2], dd[0], dd[1], dd[2]);
     SCIHPC_CHECK_LAUNCH();
-    return true;
+    return way;
   }
 
   // derivatives of f along every real axis: UCCD by (u, v, w) or CCD
   void compact(const double *f, bool upwind, double *d1[3], double *d2[3]) {
+    LineGate gate{};
     if (seg_ok && !(twin_lines && twin_partitioned)) {
-      if (upwind ? twin_seg<4, true>(f, d1, d2) || twin_seg<2, true>(f, d1, d2) || twin_seg<1, true>(f, d1, d2)
-                 : twin_seg<4, false>(f, d1, d2) || twin_seg<2, false>(f, d1, d2) || twin_seg<1, false>(f, d1, d2))
-        return;
+      SegWay way = upwind ? twin_seg<4, true>(f, d1, d2) : twin_seg<4, false>(f, d1, d2);
+      if (way == kSegNoRoom) way = upwind ? twin_seg<2, true>(f, d1, d2) : twin_seg<2, false>(f, d1, d2);
+      if (way == kSegNoRoom) way = upwind ? twin_seg<1, true>(f, d1, d2) : twin_seg<1, false>(f, d1, d2);
+      if (way == kSegDone) return;
+      if (way == kSegPassOn) gate = LineGate{seg_state, seg_call};
     }
     LineScratch sc{};
     LineCoefs co{};
@@ -2440,8 +2603,8 @@ struct scihpc_ls {
       work += (long)g.N[(a + 1) % 3] * g.N[(a + 2) % 3] * nsys;
     }
     const unsigned nbc = ceil_div(g.total, kLsBlock);
-    if (upwind) k_compact_rhs<true><<<nbc, kLsBlock, 0, stream>>>(g, f, sc);
-    else k_compact_rhs<false><<<nbc, kLsBlock, 0, stream>>>(g, f, sc);
+    if (upwind) k_compact_rhs<true><<<nbc, kLsBlock, 0, stream>>>(g, f, sc, gate);
+    else k_compact_rhs<false><<<nbc, kLsBlock, 0, stream>>>(g, f, sc, gate);
     SCIHPC_CHECK_LAUNCH();
     if (twin_lines && twin_partitioned) {
       const int segs = 1024 / twin_lines;
@@ -2476,17 +2639,17 @@ struct scihpc_ls {
         k_twin_part<8, 17, false><<<(unsigned)blocks, 1024, 0, stream>>>(g, nsys, co, sc, cr);
       }
     } else {
-      k_twin_line<<<ceil_div(work, 64), 64, 0, stream>>>(g, nsys, co, sc);
+      k_twin_line<<<ceil_div(work, 64), 64, 0, stream>>>(g, nsys, co, sc, gate);
     }
     SCIHPC_CHECK_LAUNCH();
     double *e2[3] = {nullptr, nullptr, nullptr};
     double **dd = d2 ? d2 : e2;
     if (upwind)
       k_compact_select<true><<<nbc, kLsBlock, 0, stream>>>(g.total, g.ndim, u, v, w, sc, d1[0], d1[1], d1[2], dd[0],
-                                                           dd[1], dd[2]);
+                                                           dd[1], dd[2], gate);
     else
       k_compact_select<false><<<nbc, kLsBlock, 0, stream>>>(g.total, g.ndim, nullptr, nullptr, nullptr, sc, d1[0],
-                                                            d1[1], d1[2], dd[0], dd[1], dd[2]);
+                                                            d1[1], d1[2], dd[0], dd[1], dd[2], gate);
     SCIHPC_CHECK_LAUNCH();
   }
 
@@ -2666,6 +2829,9 @@ extern "C" int scihpc_ls_create(int ndim, int nx, int ny, int nz, double dx, dou
         SCIHPC_HIP(hipGetDevice(&dev));
         if (hipDeviceGetAttribute(&lds, hipDeviceAttributeMaxSharedMemoryPerBlock, dev) == hipSuccess && lds > 0)
           h->lds_max = lds;
+        int cu = 0;
+        if (hipDeviceGetAttribute(&cu, hipDeviceAttributeMultiprocessorCount, dev) == hipSuccess && cu > 0)
+          h->num_cu = cu;
       }
       SCIHPC_HIP(hipEventCreate(&h->ev0));
       SCIHPC_HIP(hipEventCreate(&h->ev1));
@@ -2700,6 +2866,7 @@ extern "C" int scihpc_ls_destroy(scihpc_ls *h) {
                       h->seg_rows[a][2]})
       if (p) (void)hipFree(p);
   if (h->carry) (void)hipFree(h->carry);
+  if (h->seg_state) (void)hipFree(h->seg_state);
   for (auto &axis : h->ls_scr)
     for (double *p : axis)
       if (p) (void)hipFree(p);
@@ -2797,6 +2964,20 @@ extern "C" int scihpc_ls_set_line_solver(scihpc_ls *h, int partitioned) {
     ls_check(h);
     SCIHPC_REQUIRE(partitioned == 0 || partitioned == 1, "partitioned must be 0 or 1");
     h->twin_partitioned = partitioned != 0;
+  });
+}
+
+extern "C" int scihpc_ls_line_sweeps(scihpc_ls *h, long long *segmented, long long *end_to_end) {
+  return guarded([&] {
+    ls_check(h);
+    SCIHPC_REQUIRE(segmented && end_to_end, "null argument");
+    unsigned state[2] = {0, 0};
+    if (h->seg_state) {
+      SCIHPC_HIP(hipMemcpyAsync(state, h->seg_state, sizeof(state), hipMemcpyDeviceToHost, h->stream));
+      SCIHPC_HIP(hipStreamSynchronize(h->stream));
+    }
+    *segmented = h->seg_groups;
+    *end_to_end = state[1];
   });
 }
 
