@@ -2408,10 +2408,8 @@ struct scihpc_ls {
   unsigned *seg_state = nullptr;  // TwinPlan::state
   unsigned seg_call = 0;          // segmented calls so far (never 0 in one)
   long long seg_groups = 0;       // their workgroups
-  bool seg_lds_set[2][3] = {};  // k_twin_seg<LINES, UP> has been allowed its dynamic LDS, [UP][LINES / 2]
   int lds_max = 65536;      // LDS bytes a workgroup may hold on this device
   int num_cu = 256;         // compute units
-  size_t twin_lds_set = 0;  // dynamic LDS the partitioned kernels have been allowed
 
   void ensure_iface() {
     if (sgn) return;
@@ -2566,11 +2564,10 @@ struct scihpc_ls {
     pl.call = ++seg_call;
     pl.pass_on = way == kSegPassOn;
     seg_groups += total;
-    if (lds > 65536 && !seg_lds_set[UP][LINES / 2]) {
+    // the allowance is the function's, not the handle's: always the same, the most any handle needs
+    if (lds > 65536)
       SCIHPC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_twin_seg<LINES, UP>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-      seg_lds_set[UP][LINES / 2] = true;
-    }
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, lds_max - 1024));
     double *none[3] = {nullptr, nullptr, nullptr};
     double **dd = d2 ? d2 : none;
     k_twin_seg<LINES, UP><<<(unsigned)total, 64 * NS * pl.waves, lds, stream>>>(g, f, u, v, w, tb, pl, d1[0], d1[1],
@@ -2622,13 +2619,9 @@ struct scihpc_ls {
       for (int a = 0; a < g.ndim; ++a) nmax = std::max(nmax, g.N[a]);
       const size_t lds = sizeof(double) * 12 * (size_t)nmax;  // + at most 24 KiB static
       if (twin_len == 9 && lds + 24576 <= (size_t)lds_max) {
-        if (lds > twin_lds_set) {
-          SCIHPC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_twin_part<16, 9, true>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-          SCIHPC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_twin_part<8, 9, true>),
-                                         hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds));
-          twin_lds_set = lds;
-        }
+        SCIHPC_HIP(hipFuncSetAttribute(twin_lines == 16 ? reinterpret_cast<const void *>(&k_twin_part<16, 9, true>)
+                                                        : reinterpret_cast<const void *>(&k_twin_part<8, 9, true>),
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds_max - 24576));
         if (twin_lines == 16) k_twin_part<16, 9, true><<<(unsigned)blocks, 1024, lds, stream>>>(g, nsys, co, sc, cr);
         else k_twin_part<8, 9, true><<<(unsigned)blocks, 1024, lds, stream>>>(g, nsys, co, sc, cr);
       } else if (twin_lines == 16) {

@@ -2509,9 +2509,9 @@ struct scihpc_mg {
 
   template <typename T, int DIM, int P, int NT>
   void block_launch(const BlockArgs<T> &B, size_t bytes) {
-    if (bytes > 65536)
+    if (bytes > 65536)  // the function's, not the handle's: always the same
       SCIHPC_HIP(hipFuncSetAttribute(reinterpret_cast<const void *>(&k_block_vcycle<T, DIM, P, NT>),
-                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)bytes));
+                                     hipFuncAttributeMaxDynamicSharedMemorySize, (int)lds_max));
     k_block_vcycle<T, DIM, P, NT><<<1, NT, bytes, stream>>>(B);
     SCIHPC_CHECK_LAUNCH();
   }

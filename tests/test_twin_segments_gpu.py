@@ -103,3 +103,25 @@ def test_failed_call_passes_on(oracle):
             _check(oracle, ls, ndim, n, h, vel, f, upwind)
             seg, whole = (b - a for a, b in zip(before, ls.line_sweeps()))
             assert seg > 0 and (whole > 0) == (kind == "step")
+
+
+@pytest.mark.parametrize("solver", ["sequential", "partitioned"])
+def test_handles_of_different_lengths_in_turn(oracle, solver):
+    """the kernels' LDS allowance belongs to the function: a handle of shorter
+    lines must not lower it for one of longer lines"""
+    shapes = [(1024, 10, 1), (600, 10, 1)]
+    hs = [_handle(n) for n in shapes]
+    want = [None, None]
+    for ls, *_ in hs:
+        ls.set_line_solver(solver)
+    for turn in range(2):
+        for q, (ls, ndim, h, shp, _, vel) in enumerate(hs):
+            f = np.ascontiguousarray(_field("random", shp, np.random.default_rng(q)))
+            print(f"in turn {shapes[q]} {solver}", flush=True)
+            if solver == "sequential":
+                for upwind in (True, False):
+                    _check(oracle, ls, ndim, shapes[q], h, vel, f, upwind)
+                continue
+            got = ls.compact_derivatives(f, True)[0]
+            assert want[q] is None or np.array_equal(got, want[q])
+            want[q] = got
