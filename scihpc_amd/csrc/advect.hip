@@ -305,7 +305,10 @@ __device__ __forceinline__ double weno_rcp(double d) {
   return __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
 }
 
-// weno_face(a, b, c, d, e, left-biased): the value right of c
+// weno_face(a, b, c, d, e, left-biased): the value right of c.  Next to a flat
+// stencil a weight is tau / eps: from values of 1e100 on the numerator
+// overflows, where the normalised weights (WIDE) don't before 1e145.
+template <bool WIDE>
 __device__ __forceinline__ double weno_face_left(double a, double b, double c, double d, double e) {
   const double p0 = a - 2.0 * b + c, q0 = a - 4.0 * b + 3.0 * c;
   const double p1 = b - 2.0 * c + d, q1 = b - d;
@@ -318,16 +321,19 @@ __device__ __forceinline__ double weno_face_left(double a, double b, double c, d
   const double a0 = 1.0 + tau * weno_rcp(eps + b0);
   const double a1 = 6.0 + 6.0 * tau * weno_rcp(eps + b1);
   const double a2 = 3.0 + 3.0 * tau * weno_rcp(eps + b2);
-  const double num = a0 * (2.0 * a - 7.0 * b + 11.0 * c) + a1 * (5.0 * c - b + 2.0 * d) + a2 * (2.0 * c + 5.0 * d - e);
+  const double v0 = 2.0 * a - 7.0 * b + 11.0 * c, v1 = 5.0 * c - b + 2.0 * d, v2 = 2.0 * c + 5.0 * d - e;
   const double den = 6.0 * (a0 + a1 + a2);
-  const double r = weno_rcp(den), q = num * r;
+  const double r = weno_rcp(den);
+  if (WIDE) return (a0 * r) * v0 + (a1 * r) * v1 + (a2 * r) * v2;
+  const double num = a0 * v0 + a1 * v1 + a2 * v2, q = num * r;
   return __builtin_fma(__builtin_fma(-den, q, num), r, q);
 }
 
 // upwinded value right of f[2] from f[0..5]; vel: the two cells' velocities
+template <bool WIDE = false>
 __device__ __forceinline__ double weno_upwind(const double (&f)[6], double vl, double vr) {
   const bool left = vl + vr > 0.0;
-  return weno_face_left(left ? f[0] : f[5], left ? f[1] : f[4], left ? f[2] : f[3], left ? f[3] : f[2],
+  return weno_face_left<WIDE>(left ? f[0] : f[5], left ? f[1] : f[4], left ? f[2] : f[3], left ? f[3] : f[2],
                         left ? f[4] : f[1]);
 }
 
@@ -389,6 +395,7 @@ __global__ void __launch_bounds__(DIM == 3 ? kWave *kRkRows : kLsBlock)
 #pragma unroll
   for (int q = 0; q < 6; ++q) f[q] = in[p + (q - 3) * sx];
   double lower = weno_upwind(f, u[p - sx], uc);
+  if (!(fabs(lower) < __builtin_inf())) lower = weno_upwind<true>(f, u[p - sx], uc);
 #pragma unroll
   for (int q = 0; q < 5; ++q) f[q] = f[q + 1];
   for (int i = i0; i < i1; ++i, p += sx) {
@@ -397,14 +404,25 @@ __global__ void __launch_bounds__(DIM == 3 ? kWave *kRkRows : kLsBlock)
 #pragma unroll
     for (int q = 0; q < 6; ++q) a[q] = q == 2 ? f[2] : in[p + q - 2];
     const double vl = vc[p], ur = u[p + sx];
-    const double fc = weno_upwind(a, vl, vc[p + 1]);
-    const double upper = weno_upwind(f, uc, ur);
+    double fc = weno_upwind(a, vl, vc[p + 1]);
+    double upper = weno_upwind(f, uc, ur);
     double fr = 0.0, vr = 0.0;
     if constexpr (DIM == 3) {
 #pragma unroll
       for (int q = 0; q < 6; ++q) a[q] = q == 2 ? f[2] : in[p + (q - 2) * sr];
       vr = v[p];
       fr = weno_upwind(a, vr, v[p + sr]);
+    }
+    // one test for all faces, after them: a branch between them would keep
+    // their chains apart (a step 2 % slower)
+    if (!(fabs(fc) + fabs(upper) + fabs(fr) < __builtin_inf())) {
+      upper = weno_upwind<true>(f, uc, ur);
+      if constexpr (DIM == 3) fr = weno_upwind<true>(a, vr, v[p + sr]);
+#pragma unroll
+      for (int q = 0; q < 6; ++q) a[q] = in[p + q - 2];
+      fc = weno_upwind<true>(a, vl, vc[p + 1]);
+    }
+    if constexpr (DIM == 3) {
       yf[i & 1][row][lane] = fr;
       __syncthreads();
     }

@@ -54,6 +54,37 @@ def test_fused_stage_matches_oracle(oracle, n, bc):
         assert np.abs(got[at] - want[at]).max() < 1e-13 * big
 
 
+@pytest.mark.parametrize("n", [(33, 63, 1), (6, 7, 13)], ids=lambda n: "x".join(map(str, n)))
+@pytest.mark.parametrize("kind,scale", [("steps", 1e60), ("steps", 1e100), ("steps", 1e140), ("random", 2e152)])
+def test_fused_stage_at_any_magnitude(oracle, n, kind, scale):
+    """fields of two values, whose weights next to a flat stencil are their
+    differences squared over 1e-8, and fields whose squares nearly overflow
+    (up to 13 (4 s)^2 + 3 (8 s)^2 = 1.6e307 for s = 2e152; periodic, as a flat
+    stencil at a wall makes the weights themselves overflow from s = 1e149 on):
+    finite where the normalised weights are.  Same bar."""
+    ndim = 2 if n[2] == 1 else 3
+    h = (1.0 / n[0], 0.8 / n[1], 1.1 / n[2])
+    shp = padded_shape(ndim, *n)
+    rng = np.random.default_rng(sum(n))
+    phi = scale * (np.where(rng.random(shp) < 0.5, 1.0, -1.0) if kind == "steps" else rng.uniform(-1, 1, shp))
+    vel = [rng.standard_normal(shp) for _ in range(3)]
+    dt = 0.05 * min(h[:ndim])
+    print(f"fused stage {n} {kind} {scale:g}", flush=True)
+    bc = "periodic" if kind == "random" else "neumann"
+    ls = LevelSet(ndim, *n, *h, [bc] * 6)
+    ls.set_phi(phi)
+    ls.set_velocity(*vel)
+    ls.tvd_rk3(dt, 2)
+    want = phi.ravel().copy()
+    tmp = [np.zeros(want.size) for _ in range(3)]
+    types = np.full(6, BC_CODES[bc], np.int32)
+    oracle.lib.orc_tvd_rk3_weno(ndim, *n, *h, dt, types, np.zeros(6), want, *[a.ravel() for a in vel], *tmp, 2)
+    inner = tuple(slice(3, -3) if a < ndim else slice(None) for a in range(3))
+    got, want = ls.phi()[inner], want.reshape(shp)[inner]
+    assert np.isfinite(want).all()
+    assert np.abs(got / scale - want / scale).max() < 1e-13 * np.abs(want / scale).max()
+
+
 @pytest.mark.parametrize("bc", BCS, ids=lambda b: "-".join(x[:3] for x in b[:4]))
 @pytest.mark.parametrize("n", [(3, 4, 1), (33, 63, 1), (40, 1, 1), (6, 7, 5)], ids=lambda n: "x".join(map(str, n)))
 def test_uccd_stage_fills_its_ghosts(oracle, n, bc):
