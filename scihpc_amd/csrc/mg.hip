@@ -2613,7 +2613,7 @@ struct scihpc_mg {
         rr3(lv, l);
       } else {
         for (int s = 0; s < nu1; ++s) sweep(lv[l], 0, s == 0 ? z : 0);
-        if (ndim == 3 && lv[l + 1].deg / lv[l].deg == 2) rr3(lv, l);
+        if (tiled3d && ndim == 3 && lv[l + 1].deg / lv[l].deg == 2) rr3(lv, l);
         else residual_restrict(lv[l], lv[l + 1]);
       }
     }

@@ -30,7 +30,7 @@ CASES = [
     (3, (24, 24, 24), (1 / 24, 1 / 24, 1 / 24), "dirichlet", False),
     (3, (16, 16, 32), (1 / 16, 1 / 16, 1 / 16), "neumann", True),
     (2, (54, 54, 1), (1 / 54, 1 / 54, 1.0), "neumann", False),  # ratio-3 coarsening
-    # z-streaming 3-D sweeps on levels 0 and 1 (density and face coefficients)
+    # 3-D tiles on level 0 (density), colour kernels and the one-workgroup cycle below
     (3, (32, 32, 32), (1 / 32, 1 / 32, 1 / 32), "neumann", True),
     (3, (32, 48, 32), (1 / 32, 1 / 32, 1 / 32), "dirichlet", False),
 ]
@@ -252,10 +252,12 @@ def test_errors_are_status_codes():
 @pytest.mark.parametrize("case", [c for c in CASES if c[0] == 3],
                          ids=lambda c: f"{c[1]}-{c[3]}-{'var' if c[4] else 'const'}")
 @pytest.mark.parametrize("precision", [PREC_FP64, PREC_MIXED], ids=["fp64", "mixed"])
-def test_z3_sweeps_match_colour_kernels(oracle, case, precision, monkeypatch):
-    """The z-streaming 3-D sweep is the same red-black Gauss-Seidel as the
-    two colour kernels: equal V-cycle iterates (FP64 to rounding) and equal
-    solve results."""
+def test_3d_tiles_match_colour_kernels(oracle, case, precision, monkeypatch):
+    """The 3-D tile kernels (k_pre3d, k_post3d; and the density restriction of
+    a first cycle from a non-zero iterate) are the same red-black Gauss-Seidel
+    as the two colour kernels with the generic restriction: equal V-cycle
+    iterates (FP64 to rounding) and equal solve results.  (The z-marching
+    sweeps, on levels of over 2^18 cells: test_mg_production_gpu.py.)"""
     rng = np.random.default_rng(7)
     sols, stats = [], []
     for flag in ("1", "0"):

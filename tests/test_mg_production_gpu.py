@@ -161,12 +161,17 @@ def test_fcg_iterates_match_oracle(oracle, case, monkeypatch):
     assert sm["converged"] and sm["cycles"] <= it + 1, (sm, it)
 
 
-# 3-D: z-marching kernels on levels of 2^18 cells and more
+# 3-D: z-marching restriction and direction on levels of 2^18 cells and more,
+# z-marching sweeps and prolongation above; ragged tiles and plane chunks, and
+# (last) a level 1 whose sweeps read face coefficients
 CASES_3D = [
     ("var-plane-64^3", (64, 64, 64), "neumann", True),
     ("var-plane-64x64x128", (64, 64, 128), "neumann", True),
     ("dir-64x64x128", (64, 64, 128), "dirichlet", False),
     ("neu-const-64^3", (64, 64, 64), "neumann", False),
+    ("var-plane-80x72x56", (80, 72, 56), "neumann", True),
+    ("dir-88x72x56", (88, 72, 56), "dirichlet", False),
+    ("var-plane-144x144x112", (144, 144, 112), "neumann", True),
 ]
 
 
