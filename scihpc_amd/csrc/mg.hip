@@ -4421,6 +4421,7 @@ extern "C" int scihpc_mg_time_kernel(scihpc_mg *h, int which, int iters, double 
     const double n = (double)l0.n, nc = (double)h->d[1].n;
     const double nf = h->variable ? h->ndim : 0;  // face arrays per level
     const bool tiled = h->fused_level(h->d, 0);
+    const bool tile3 = !tiled && h->tile3_level(h->d, 0);
     const bool z3 = !tiled && h->z3_level(h->d, 0) && h->d[1].deg == 2;
     // coefficient arrays a level-0 sweep reads: rho (z-streaming, A(rho)), faces, none
     const double na = z3 ? (h->variable ? 1.0 : 0.0) : nf;
@@ -4430,18 +4431,26 @@ extern "C" int scihpc_mg_time_kernel(scihpc_mg *h, int which, int iters, double 
     oa.p_new = h->p_alt;
     oa.r32 = f0.rhs_alt;
     auto pre = [&](auto &lv) {
+      if (tile3) {  // from a zero iterate
+        h->pre3d(lv, 0, 2);
+        return;
+      }
       for (int s = 0; s < 2; ++s) {
         if (z3) h->sweep3(lv, 0, 0, 0);
         else h->sweep(lv[0], 0, 0);
       }
-      if (z3) h->rr3(lv, 0);
+      if (h->tiled3d && h->ndim == 3 && h->d[1].deg == 2) h->rr3(lv, 0);
       else h->residual_restrict(lv[0], lv[1]);
     };
     auto post = [&](auto &lv, int mode) {
-      h->prolong_add(lv[1], lv[0]);
-      for (int s = 0; s < 2; ++s) {
-        if (z3) h->sweep3(lv, 0, 1, 0);
-        else h->sweep(lv[0], 1, 0);
+      if (tile3) {
+        h->post3d(lv, 0, 2);
+      } else {
+        h->prolong_add(lv[1], lv[0]);
+        for (int s = 0; s < 2; ++s) {
+          if (z3) h->sweep3(lv, 0, 1, 0);
+          else h->sweep(lv[0], 1, 0);
+        }
       }
       h->post0_generic(lv, mode, oa);
     };
@@ -4502,8 +4511,11 @@ extern "C" int scihpc_mg_time_kernel(scihpc_mg *h, int which, int iters, double 
       // sweep (3 + na) s N; residual + restriction (2 + na) s N + 2 s Nc;
       // prolong-add 2 s N + s Nc; FP64 outer update (32 + 8 nf) N;
       // FP64 residual norm (16 + 8 nf) N
+      // (3-D tiles: right-hand side, faces and the iterate once, coarse level)
       const double sd = which == 1 || which == 2 ? 4.0 : 8.0;
-      if (which <= 1) b = 2.0 * (3.0 + na) * sd * n + (2.0 + na) * sd * n + 2.0 * sd * nc;
+      if (tile3 && which <= 1) b = (2.0 + nf) * sd * n + 2.0 * sd * nc;
+      else if (tile3) b = (3.0 + nf) * sd * n + sd * nc + (which == 2 ? (32.0 + 8.0 * nf) * n : (16.0 + 8.0 * nf) * n);
+      else if (which <= 1) b = 2.0 * (3.0 + na) * sd * n + (2.0 + na) * sd * n + 2.0 * sd * nc;
       else
         b = 2.0 * sd * n + sd * nc + 2.0 * (3.0 + na) * sd * n +
             (which == 2 ? (32.0 + 8.0 * nf) * n : (16.0 + 8.0 * nf) * n);

@@ -329,6 +329,9 @@ def test_timing_hooks(ndim):
         assert math.isfinite(ms) and ms > 0 and b > 0
     assert g.time_kernel(4, iters=1)[1] == 16.0 * cells + 8.0 * coarse
     assert g.time_kernel(5, iters=1)[1] == (2 + ndim) * 8.0 * cells
+    if ndim == 3:  # the tiles the solve runs on this level: one launch each way
+        assert g.time_kernel(1, iters=1)[1] == (2 + ndim) * 4.0 * cells + 2 * 4.0 * coarse
+        assert g.time_kernel(3, iters=1)[1] == (3 + ndim) * 8.0 * cells + 8.0 * coarse + (2 + ndim) * 8.0 * cells
     if ndim == 2:  # the fused FCG update + pre-smoothing, on the last mixed FCG solve's vectors
         ms, b = g.time_kernel(6, iters=2)
         assert math.isfinite(ms) and ms > 0 and b == (4 * ndim + 56) * cells + 8.0 * coarse
