@@ -293,8 +293,11 @@ __global__ void __launch_bounds__(kLsBlock) k_bc_axis_fields(Grid g, BcFields m,
 // What bounds it: FP64 issue.  A face took ten IEEE divisions (about 14
 // instructions each) and was formed by both its cells; here it takes four
 // reciprocals (v_rcp_f64 and two Newton steps).  The WENO-Z weights are
-// ratios, so their common denominator is left out and one division by the
-// weights' sum remains, its quotient corrected by its remainder.
+// ratios, so their common denominator is left out; the reciprocal of their sum
+// is applied to them before the values are, as next to a flat stencil a weight
+// is a squared difference over 1e-8 (from values of 1e100 on its product
+// overflows; as many operations as one corrected quotient, and over 14 grids
+// its error against 64 bits 1.011e-16, the divisions' 1.016e-16).
 // Measured at 1024 x 512: a stage with its boundary conditions 20.3 + 2 x 4.7
 // us in three launches before, 11.9 us here (a step 81 -> 36 us).
 constexpr int kRkRows = 8;
@@ -305,10 +308,7 @@ __device__ __forceinline__ double weno_rcp(double d) {
   return __builtin_fma(r, __builtin_fma(-d, r, 1.0), r);
 }
 
-// weno_face(a, b, c, d, e, left-biased): the value right of c.  Next to a flat
-// stencil a weight is tau / eps: from values of 1e100 on the numerator
-// overflows, where the normalised weights (WIDE) don't before 1e145.
-template <bool WIDE>
+// weno_face(a, b, c, d, e, left-biased): the value right of c
 __device__ __forceinline__ double weno_face_left(double a, double b, double c, double d, double e) {
   const double p0 = a - 2.0 * b + c, q0 = a - 4.0 * b + 3.0 * c;
   const double p1 = b - 2.0 * c + d, q1 = b - d;
@@ -324,16 +324,13 @@ __device__ __forceinline__ double weno_face_left(double a, double b, double c, d
   const double v0 = 2.0 * a - 7.0 * b + 11.0 * c, v1 = 5.0 * c - b + 2.0 * d, v2 = 2.0 * c + 5.0 * d - e;
   const double den = 6.0 * (a0 + a1 + a2);
   const double r = weno_rcp(den);
-  if (WIDE) return (a0 * r) * v0 + (a1 * r) * v1 + (a2 * r) * v2;
-  const double num = a0 * v0 + a1 * v1 + a2 * v2, q = num * r;
-  return __builtin_fma(__builtin_fma(-den, q, num), r, q);
+  return (a0 * r) * v0 + (a1 * r) * v1 + (a2 * r) * v2;
 }
 
 // upwinded value right of f[2] from f[0..5]; vel: the two cells' velocities
-template <bool WIDE = false>
 __device__ __forceinline__ double weno_upwind(const double (&f)[6], double vl, double vr) {
   const bool left = vl + vr > 0.0;
-  return weno_face_left<WIDE>(left ? f[0] : f[5], left ? f[1] : f[4], left ? f[2] : f[3], left ? f[3] : f[2],
+  return weno_face_left(left ? f[0] : f[5], left ? f[1] : f[4], left ? f[2] : f[3], left ? f[3] : f[2],
                         left ? f[4] : f[1]);
 }
 
@@ -395,7 +392,6 @@ __global__ void __launch_bounds__(DIM == 3 ? kWave *kRkRows : kLsBlock)
 #pragma unroll
   for (int q = 0; q < 6; ++q) f[q] = in[p + (q - 3) * sx];
   double lower = weno_upwind(f, u[p - sx], uc);
-  if (!(fabs(lower) < __builtin_inf())) lower = weno_upwind<true>(f, u[p - sx], uc);
 #pragma unroll
   for (int q = 0; q < 5; ++q) f[q] = f[q + 1];
   for (int i = i0; i < i1; ++i, p += sx) {
@@ -404,25 +400,14 @@ __global__ void __launch_bounds__(DIM == 3 ? kWave *kRkRows : kLsBlock)
 #pragma unroll
     for (int q = 0; q < 6; ++q) a[q] = q == 2 ? f[2] : in[p + q - 2];
     const double vl = vc[p], ur = u[p + sx];
-    double fc = weno_upwind(a, vl, vc[p + 1]);
-    double upper = weno_upwind(f, uc, ur);
+    const double fc = weno_upwind(a, vl, vc[p + 1]);
+    const double upper = weno_upwind(f, uc, ur);
     double fr = 0.0, vr = 0.0;
     if constexpr (DIM == 3) {
 #pragma unroll
       for (int q = 0; q < 6; ++q) a[q] = q == 2 ? f[2] : in[p + (q - 2) * sr];
       vr = v[p];
       fr = weno_upwind(a, vr, v[p + sr]);
-    }
-    // one test for all faces, after them: a branch between them would keep
-    // their chains apart (a step 2 % slower)
-    if (!(fabs(fc) + fabs(upper) + fabs(fr) < __builtin_inf())) {
-      upper = weno_upwind<true>(f, uc, ur);
-      if constexpr (DIM == 3) fr = weno_upwind<true>(a, vr, v[p + sr]);
-#pragma unroll
-      for (int q = 0; q < 6; ++q) a[q] = in[p + q - 2];
-      fc = weno_upwind<true>(a, vl, vc[p + 1]);
-    }
-    if constexpr (DIM == 3) {
       yf[i & 1][row][lane] = fr;
       __syncthreads();
     }
