@@ -287,9 +287,10 @@ __global__ void __launch_bounds__(kLsBlock) k_bc_axis_fields(Grid g, BcFields m,
 // k_rk3_stage<1>'s work with every face value formed once and the ghosts
 // filled by the cells they copy.  The last axis is contiguous: a wavefront
 // takes 64 faces and so 63 cells of a row, each lane handing its face to the
-// next.  Threads march `run` cells along the first axis and carry the face
-// between them.  In 3-D a workgroup is kRkRows rows of the middle axis, the
-// lowest of which only forms faces for the row above it.
+// next, or several short rows (SHORT: `lanes` lanes each).  Threads march `run`
+// cells along the first axis and carry the face between them.  In 3-D a
+// workgroup's eight wavefronts hold rows of the middle axis, the lowest of
+// which only forms faces for the row above it.
 // What bounds it: FP64 issue.  A face took ten IEEE divisions (about 14
 // instructions each) and was formed by both its cells; here it takes four
 // reciprocals (v_rcp_f64 and two Newton steps).  The WENO-Z weights are
@@ -364,26 +365,29 @@ __device__ __forceinline__ void ghosts_of(const BcSpec &bc, int a, int n, double
   }
 }
 
-template <int DIM, int STAGE>
+template <int DIM, int STAGE, bool SHORT>
 __global__ void __launch_bounds__(DIM == 3 ? kWave *kRkRows : kLsBlock)
     k_rk3_fused(Grid g, const double *__restrict__ in, double *__restrict__ out, const double *__restrict__ u,
                 const double *__restrict__ v, const double *__restrict__ w, double *__restrict__ s1,
                 double *__restrict__ s2, double dt, BcSpec bc, int ghosts, int tiles_c, int tiles_r,
-                int run) {
+                int run, int lanes) {
   constexpr int C = DIM - 1;  // the contiguous axis
-  __shared__ double yf[DIM == 3 ? 2 : 1][DIM == 3 ? kRkRows : 1][kWave];
-  const int lane = (int)threadIdx.x % kWave, row = (int)threadIdx.x / kWave;
-  // 2-D: every wavefront has a tile of its own
-  int tile = DIM == 3 ? (int)blockIdx.x : (int)blockIdx.x * (kLsBlock / kWave) + row;
+  __shared__ double yf[DIM == 3 ? 2 : 1][DIM == 3 ? kRkRows * kWave : 1];
+  const int width = SHORT ? lanes : kWave;
+  const int sub = kWave / width, part = (int)threadIdx.x % kWave / width;  // rows a wavefront, this lane's
+  const int lane = (int)threadIdx.x % kWave - part * width, row = (int)threadIdx.x / kWave * sub + part;
+  const bool spare = part >= sub;  // a lane too many
+  // 2-D: every row of a wavefront has a tile of its own
+  int tile = DIM == 3 ? (int)blockIdx.x : (int)blockIdx.x * (kLsBlock / kWave) * sub + row;
   const int tc = tile % tiles_c;
   tile /= tiles_c;
   const int tr = DIM == 3 ? tile % tiles_r : 0;
   if (DIM == 3) tile /= tiles_r;
   const int i0 = tile * run, i1 = min(g.n[0], i0 + run);
-  if (DIM == 2 && i0 >= g.n[0]) return;  // whole wavefronts, no barrier in 2-D
+  if (DIM == 2 && (spare || i0 >= g.n[0])) return;  // whole rows, no barrier in 2-D
   const int nc = g.n[C], nr = DIM == 3 ? g.n[1] : 1;
-  const int c = tc * (kWave - 1) + lane - 1, r = DIM == 3 ? tr * (kRkRows - 1) + row - 1 : 0;
-  const bool own = lane > 0 && c < nc && (DIM == 2 || (row > 0 && r < nr));  // lane 0 and row 0 form faces only
+  const int c = tc * (width - 1) + lane - 1, r = DIM == 3 ? tr * (kRkRows * sub - 1) + row - 1 : 0;
+  const bool own = !spare && lane > 0 && c < nc && (DIM == 2 || (row > 0 && r < nr));  // lane 0 and row 0 form faces only
   const int cc = min(c, nc - 1), rc = min(r, nr - 1);
   const long sx = g.s[0], sr = g.s[1];
   const double *vc = DIM == 3 ? w : v;
@@ -408,13 +412,13 @@ __global__ void __launch_bounds__(DIM == 3 ? kWave *kRkRows : kLsBlock)
       for (int q = 0; q < 6; ++q) a[q] = q == 2 ? f[2] : in[p + (q - 2) * sr];
       vr = v[p];
       fr = weno_upwind(a, vr, v[p + sr]);
-      yf[i & 1][row][lane] = fr;
+      if (!spare) yf[i & 1][row * width + lane] = fr;
       __syncthreads();
     }
     const double fl = __shfl_up(fc, 1, kWave);
     if (own) {
       double s = -uc * ((upper - lower) / g.h[0]);
-      if constexpr (DIM == 3) s -= vr * ((fr - yf[i & 1][row - 1][lane]) / g.h[1]);
+      if constexpr (DIM == 3) s -= vr * ((fr - yf[i & 1][(row - 1) * width + lane]) / g.h[1]);
       s -= vl * ((fc - fl) / g.h[C]);
       const double x = f[2];
       double y;
@@ -2747,6 +2751,46 @@ struct scihpc_ls {
     redist_stage<DIM, 3>(b, f, dt, rdt);
   }
 
+  // k_rk3_fused's shape for this grid: rows a wavefront, tiles across the
+  // last and the middle axis, cells a march
+  struct RkPlan {
+    int sub = 0, tc = 0, tr = 0, run = 0;
+  } rk;
+  template <int DIM>
+  const RkPlan &rk_plan() {
+    if (rk.sub) return rk;
+    // Several short rows a wavefront where that takes under 0.8 of the
+    // wavefronts (a last axis of few cells, or of few more than a multiple of
+    // 63) and those are several for every SIMD: on smaller grids a launch's
+    // latency counts, which it lengthens (32^3 18 -> 20 us a step).
+    // Microseconds a step, one row / several / a thread a cell with the ghosts
+    // apart: 600 x 16 x 16 90 / 39 / 82, with Dirichlet sides 136 / 87 /
+    // 101; 256 x 16 x 64 72 / 54 / 92, Dirichlet 126 / 105 / 111; 80 x 70 x 90
+    // 97 / 62 / 128, 128^3 (0.74) 236 / 211 / 351, 128 x 128 x 33 101 / 82 / 135.
+    const int nc = g.n[DIM - 1];
+    auto tiles_c = [&](int q) { return (int)ceil_div(nc, kWave / q - 1); };
+    auto tiles_r = [&](int q) { return DIM == 3 ? (int)ceil_div(g.n[1], kRkRows * q - 1) : 1; };
+    auto cost = [&](int q) { return (DIM == 3 ? 1.0 : 1.0 / q) * tiles_c(q) * tiles_r(q); };
+    rk.sub = 1;
+    for (int q = 2; q <= 8 && cost(1) * g.n[0] * (DIM == 3 ? kRkRows : 1) >= 16.0 * num_cu; ++q)
+      if (cost(q) < 0.8 * cost(1) && cost(q) < cost(rk.sub)) rk.sub = q;
+    rk.tc = tiles_c(rk.sub);
+    rk.tr = tiles_r(rk.sub);
+    // cells a march: a wavefront forms DIM faces a cell and one more, so
+    // long marches form fewer, but the 1024 SIMDs want two or three
+    // wavefronts each to hide their chains.  Microseconds a step measured with
+    // 1 / 2 / 3 / 4 / 6 / 8 cells: 1024 x 512 42 / 39 / 36 / 39 / 40 / 48,
+    // 333 x 501 21 / 22 / 22 / 24 / 29 / 35, 2048^2 264 / 188 / 163 / 157 /
+    // 145 / 146, 128^3 (one row) 356 / 273 / 245 / 246 / 224 / 231.
+    rk.run = 6;
+    auto waves = [&](int q) {
+      const long t = (long)rk.tc * rk.tr * ceil_div(g.n[0], q);
+      return DIM == 3 ? t * kRkRows : t / rk.sub;
+    };
+    while (rk.run > 1 && waves(rk.run) < 4L * num_cu * (DIM == 3 ? 3 : 5) / 2) --rk.run;
+    return rk;
+  }
+
   // one WENO stage with its boundary conditions: in the stage's kernel but
   // for Dirichlet sides, which change boundary cells other axes read
   template <int DIM, int STAGE>
@@ -2757,20 +2801,16 @@ struct scihpc_ls {
       apply_bc(out, -1);
     } else {
       const bool dir = dirichlet();
-      const int tc = (int)ceil_div(g.n[DIM - 1], kWave - 1), tr = DIM == 3 ? (int)ceil_div(g.n[1], kRkRows - 1) : 1;
-      // cells a march: a wavefront forms DIM faces a cell and one more, so
-      // long marches form fewer, but the 1024 SIMDs want two or three
-      // wavefronts each to hide their chains.  Microseconds a step measured with
-      // 1 / 2 / 3 / 4 / 6 / 8 cells: 1024 x 512 42 / 39 / 36 / 39 / 40 / 48,
-      // 333 x 501 21 / 22 / 22 / 24 / 29 / 35, 2048^2 264 / 188 / 163 / 157 /
-      // 145 / 146, 128^3 356 / 273 / 245 / 246 / 224 / 231.
-      int run = 6;
-      auto waves = [&](int q) { return (long)tc * tr * ceil_div(g.n[0], q) * (DIM == 3 ? kRkRows : 1); };
-      while (run > 1 && waves(run) < (DIM == 3 ? 1536 : 2560)) --run;
-      const long tiles = (long)tc * tr * ceil_div(g.n[0], run);
-      constexpr int per = DIM == 3 ? 1 : kLsBlock / kWave;
-      k_rk3_fused<DIM, STAGE><<<ceil_div(tiles, per), DIM == 3 ? kWave * kRkRows : kLsBlock, 0, stream>>>(
-          g, in, out, u, v, w, s1, s2, dt, bc, dir ? 0 : 1, tc, tr, run);
+      const RkPlan &pl = rk_plan<DIM>();
+      const long tiles = (long)pl.tc * pl.tr * ceil_div(g.n[0], pl.run);
+      const int per = DIM == 3 ? 1 : kLsBlock / kWave * pl.sub;
+      const unsigned nb = ceil_div(tiles, per), nt = DIM == 3 ? kWave * kRkRows : kLsBlock;
+      if (pl.sub > 1)
+        k_rk3_fused<DIM, STAGE, true><<<nb, nt, 0, stream>>>(g, in, out, u, v, w, s1, s2, dt, bc, !dir, pl.tc, pl.tr,
+                                                             pl.run, kWave / pl.sub);
+      else
+        k_rk3_fused<DIM, STAGE, false><<<nb, nt, 0, stream>>>(g, in, out, u, v, w, s1, s2, dt, bc, !dir, pl.tc, pl.tr,
+                                                              pl.run, kWave);
       SCIHPC_CHECK_LAUNCH();
       if (dir) apply_bc(out, -1);
     }

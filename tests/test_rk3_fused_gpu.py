@@ -1,6 +1,7 @@
 """The fused WENO5 TVD-RK3 stage (k_rk3_fused) against the oracle at the edges
-of its tiles: rows of 62, 63 and 64 cells and of a few, marches that end
-early, 3-D row tiles of 6, 7 and 8, and every boundary condition, mixed over
+of its tiles: rows of 62, 63 and 64 cells, several short rows a wavefront (30,
+31 and 32 cells and fewer), marches that end early, 3-D row tiles of 6, 7 and 8
+and of several short rows, and every boundary condition, mixed over
 the sides (Dirichlet sides take the separate ghost kernels).
 
 Bar: 1e-13 of the largest value after two steps; a face value is formed from
@@ -16,7 +17,8 @@ from scihpc_amd import LevelSet, padded_shape
 from scihpc_amd._capi import BC_CODES
 
 SHAPES = [(3, 4, 1), (5, 62, 1), (33, 63, 1), (20, 64, 1), (7, 127, 1), (900, 190, 1), (6, 6, 62), (9, 7, 64), (13, 8, 5),
-          (20, 15, 126)]
+          (20, 15, 126), (100, 30, 1), (7, 31, 1), (50, 32, 1), (700, 20, 1), (9, 15, 31), (5, 16, 31), (8, 23, 20),
+          (12, 24, 20), (6, 50, 9), (5, 3, 30)]
 BCS = [["neumann"] * 6, ["periodic"] * 6, ["no_slip", "slip", "neumann", "no_slip", "slip", "neumann"],
        ["dirichlet", "neumann", "slip", "dirichlet", "neumann", "dirichlet"]]
 
