@@ -291,7 +291,8 @@ __global__ void __launch_bounds__(kLsBlock) k_bc_axis_fields(Grid g, BcFields m,
 // cells along the first axis and carry the face between them.  In 3-D a
 // workgroup's eight wavefronts hold rows of the middle axis, the lowest of
 // which only forms faces for the row above it.
-// What bounds it: FP64 issue.  A face took ten IEEE divisions (about 14
+// What bounds it: FP64 issue (the VALU is active in 59 % of the cycles in
+// which a SIMD has work, at 1024 x 512).  A face took ten IEEE divisions (about 14
 // instructions each) and was formed by both its cells; here it takes four
 // reciprocals (v_rcp_f64 and two Newton steps).  The WENO-Z weights are
 // ratios, so their common denominator is left out; the reciprocal of their sum
@@ -1018,10 +1019,10 @@ __global__ void __launch_bounds__(kLsBlock)
 
 // twin_bks (matrix_solver.cpp:58-83) in place on S/SS holding the
 // right-hand sides; thread t: axis a, then line t % lines, system t / lines
-__global__ void __launch_bounds__(64) k_twin_line(Grid g, int nsys, LineCoefs co, LineScratch sc,
-                                                  LineGate gate) {
+template <bool GATE>  // (looking at a gate costs a call of long lines 3 %)
+__global__ void __launch_bounds__(64) k_twin_line(Grid g, int nsys, LineCoefs co, LineScratch sc, LineGate gate) {
 #pragma clang fp contract(off)
-  if (gate.closed()) return;
+  if (GATE && gate.closed()) return;
   constexpr int B = kLineChunk;
   long t = (long)blockIdx.x * blockDim.x + threadIdx.x;
   int a = 0;
@@ -1144,10 +1145,10 @@ __global__ void __launch_bounds__(64) k_twin_line(Grid g, int nsys, LineCoefs co
 // only the sign of a zero may differ.  Segment lengths are odd, so the 64
 // lanes of a wavefront (LINES lines x 64 / LINES segments) read different
 // banks.
-// What bounds it: the instructions a lone wavefront issues for about 240
-// steps forward and 230 backward (instead of 2 x 1030), and LDS: whole lines
-// leave one workgroup a CU, so 388 workgroups run as two rounds.  Measured at
-// 1024 x 512: 91 us, where right-hand sides, one thread a line and selection
+// What bounds it: the dependent FP64 operations of a lone wavefront for about
+// 240 steps forward and 230 backward (instead of 2 x 1030; it issues in 30 %
+// of its cycles), and LDS: whole lines leave one workgroup a CU, so 388
+// workgroups run as two rounds.  Measured at 1024 x 512: 93 us, where right-hand sides, one thread a line and selection
 // took 11.7 + 383 + 7.2 us in three launches; a UCCD TVD-RK3 step 1.24 ->
 // 0.30 ms, of a field of two values 1.24 -> 0.77 (end to end with a thread a
 // line and divisions it was 1.24).  Lines that do not fit LDS (over 4416
@@ -1517,8 +1518,9 @@ __global__ void __launch_bounds__(512)  // two systems, at most four wavefronts 
   if (alone) {
     // From end to end, two lanes a line: one holds f', the other f'', and they
     // exchange them; a wavefront on its own is bound by the instructions of a
-    // step, and this halves them.  Blocks of steps whose quotients may not be
-    // IEEE ones are done again with divisions.
+    // step, and this halves them (68 clocks a position forward and 150
+    // backward, 110 and 270 with one lane and divisions).  Blocks of steps
+    // whose quotients may not be IEEE ones are done again with divisions.
     fill();
     __syncthreads();
     if (ts < 2 * LINES) {
@@ -1853,12 +1855,13 @@ __global__ void __launch_bounds__(kLsBlock)
 #pragma clang fp contract(off)
   const long c = (long)blockIdx.x * blockDim.x + threadIdx.x;
   if (c >= g.total) return;
-  int q[3];
-  padded_ijk(g, c, q);
-  int out = 0;
+  int q[3] = {0, 0, 0}, out = 0;
+  if (ghosts) {  // (else every cell is advanced and apply_bc fills the ghosts)
+    padded_ijk(g, c, q);
 #pragma unroll
-  for (int a = 0; a < DIM; ++a) out += q[a] < g.off[a] || q[a] >= g.off[a] + g.n[a];
-  if (out == 1) return;
+    for (int a = 0; a < DIM; ++a) out += q[a] < g.off[a] || q[a] >= g.off[a] + g.n[a];
+    if (out == 1) return;
+  }
   double s = -u[c] * fx[c];
   if (DIM > 1) s -= v[c] * fy[c];
   if (DIM > 2) s -= w[c] * fz[c];
@@ -2165,7 +2168,8 @@ __global__ void __launch_bounds__(kLsBlock)
 // inner 14 x 30 positions are advanced.  The rim's gradients are formed twice
 // (512 for 420 cells), which costs less than the gradient's way through
 // memory and a launch.  What bounds it: FP64 issue, some 480 instructions a
-// position, and on small grids the chain of one wavefront.
+// position (the VALU is active in 72 % of the cycles in which a SIMD has work,
+// at 1024 x 512), and on small grids the chain of one wavefront.
 // Measured: a step's three stages at 501 x 333 65 us in twelve launches
 // before, 24 here; 64 x 128 16 us, 1024^2 74, 3000 x 2000 368.  Tiles of 8 x
 // 32 / 8 x 64 / 16 x 16: 25 / 24 / 26, 15 / 17 / 15, 79 / 78 / 77, 390 / 401
@@ -2639,7 +2643,8 @@ struct scihpc_ls {
         k_twin_part<8, 17, false><<<(unsigned)blocks, 1024, 0, stream>>>(g, nsys, co, sc, cr);
       }
     } else {
-      k_twin_line<<<ceil_div(work, 64), 64, 0, stream>>>(g, nsys, co, sc, gate);
+      if (gate.flag) k_twin_line<true><<<ceil_div(work, 64), 64, 0, stream>>>(g, nsys, co, sc, gate);
+      else k_twin_line<false><<<ceil_div(work, 64), 64, 0, stream>>>(g, nsys, co, sc, gate);
     }
     SCIHPC_CHECK_LAUNCH();
     double *e2[3] = {nullptr, nullptr, nullptr};
